@@ -16,7 +16,8 @@
 // Layout in HBM: complex buffers [L0, L1, L2, batch] (dims past the rank are
 // the batch, folded into one index), convT pairs.
 //
-// Kernels:
+// Kernels: real data of rank 2 with padded sides 64..4096 runs fft2_rows,
+// fft2_cols and fft2_rows_inv (below); everything else
 //  * fft_pad: signal or filter (any dtype) -> zero-padded complex buffer;
 //  * fft_pass: a batched radix-2 FFT of power-of-two length L <= 4096 along
 //    one axis (element stride `stride`), M transforms per 256-lane workgroup
@@ -29,63 +30,36 @@
 //  * fft_mul: spectrum product with the batch pairing (in place when the
 //    output slice is the signal's or the filter's own);
 //  * fft_crop: crop, scale and the output dtype's conversion rule.
-// Twiddles W_4096^j (j < 2048) live in a static device table per precision,
-// filled once per device by fft_twiddle_init (sincospi in double).
+// Twiddles live in static device tables per precision, filled once per device
+// by fft_twiddle_init (sincospi in double).
 #include <mutex>
+#include <type_traits>
 
-#include "kcommon.hpp"
+#include "fft_core.hpp"
 #include "../../../include/afhip_kernels.h"
 
 namespace afhip {
 
-constexpr int FFT_LMAX = 4096;        // longest in-LDS transform
 constexpr int FFT_LOGMAX = 12;
 constexpr int FFT_THREADS = 256;
 
-static __device__ float2 g_fft_tw32[FFT_LMAX / 2];
-static __device__ double2 g_fft_tw64[FFT_LMAX / 2];
-
 __global__ __launch_bounds__(256) void fft_twiddle_init() {
-    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < FFT_LMAX / 2; j += gridDim.x * blockDim.x) {
+    const int first = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    for (int j = first; j < FFT_LMAX / 2; j += step) {
         double s, c;
         sincospi(-2.0 * j / FFT_LMAX, &s, &c);
         g_fft_tw32[j] = make_float2((float)c, (float)s);
         g_fft_tw64[j] = make_double2(c, s);
     }
-}
-
-template <typename R>
-struct FT;
-template <>
-struct FT<float> {
-    typedef float2 C;
-    __device__ static C tw(int j) { return g_fft_tw32[j]; }
-    __device__ static C mk(float a, float b) { return make_float2(a, b); }
-    // W_L^m for arbitrary L (four-step twiddles), evaluated in double
-    __device__ static C wl(long long m, long long L, bool inv) {
-        double s, c;
-        sincospi((inv ? 2.0 : -2.0) * (double)m / (double)L, &s, &c);
-        return make_float2((float)c, (float)s);
+    for (int l = FFT_REG_MIN; l <= FFT_REG_MAX; ++l) {
+        const int nt = 1 << (l - 3), at = fft_reg_at(l);
+        for (int e = first; e < fft_reg_ntw(l) * nt; e += step) {
+            double s, c;
+            sincospi(-2.0 * fft_reg_angle(l, e / nt, e % nt) / (1 << l), &s, &c);
+            g_fft_lane32[at + e] = make_float2((float)c, (float)s);
+            g_fft_lane64[at + e] = make_double2(c, s);
+        }
     }
-};
-template <>
-struct FT<double> {
-    typedef double2 C;
-    __device__ static C tw(int j) { return g_fft_tw64[j]; }
-    __device__ static C mk(double a, double b) { return make_double2(a, b); }
-    __device__ static C wl(long long m, long long L, bool inv) {
-        double s, c;
-        sincospi((inv ? 2.0 : -2.0) * (double)m / (double)L, &s, &c);
-        return make_double2(c, s);
-    }
-};
-
-template <typename C>
-__device__ inline C cmul2(C a, C b) {
-    C r;
-    r.x = a.x * b.x - a.y * b.y;
-    r.y = a.x * b.y + a.y * b.x;
-    return r;
 }
 
 struct FftPass {
@@ -274,6 +248,274 @@ __global__ __launch_bounds__(256) void fft_crop(T *__restrict__ out, const typen
     }
 }
 
+// ------------------------------------------------- two-dimensional, real
+// Rank-2 convolution of real data in three launches:
+//  * fft2_rows: rows of the signal and of the filter, two real rows of one
+//    slice per complex transform, straight from the source type; writes the
+//    half spectrum (k0 = 0..L0/2) transposed, [slice][k0][row], so that the
+//    next pass reads whole columns. Rows of padding are neither transformed
+//    nor stored.
+//  * fft2_cols: per column, the filter's and the signal's transforms along
+//    dim1, their product and the inverse, all in registers; keeps the rows of
+//    the result only.
+//  * fft2_rows_inv: two result rows per inverse transform, cropped, scaled and
+//    converted.
+// 1024^2 with a 31x31 filter (padded to 2048^2): 33 us, 8.4 MB of spectrum
+// written and read twice, against 474 us for ten passes over 33.6 MB padded
+// complex arrays (12 LDS stages each). What is left is the latency of one
+// round of workgroups per launch: rows 11.5 us, columns 15 us (three
+// transforms of four passes each, four workgroups per CU), rows back 8 us.
+// Giving the columns of L0/2 and 0 one transform (1024 workgroups in place of
+// 1025) cost registers and was slower (17.4 us with three workgroups per CU,
+// 20.6 us spilled to keep four), as was sharing store lines between the row
+// pairs of a 512-lane workgroup (12.3 us).
+// Two rows share a transform only inside a slice, where a NaN or an infinity
+// reaches every output in any case.
+struct Fft2Side {
+    const void *p;      // source, [d0, d1] slices
+    long long out;      // offset of its spectrum in the workspace (elements)
+    int type, d0, d1;
+    int pairs;          // row pairs per slice
+    int pitch;          // spectrum rows per column (even)
+    unsigned ntrans;    // pairs * slices
+};
+
+// Eight points each of two rows (or of one, with zeros for the other), as
+// sixteen loads in flight at once: the type is chosen outside, and lanes past
+// the row read its last element, so no load waits behind a branch (a switch
+// and a mask per load made each wait for the one before).
+template <typename T, typename R, int NT>
+__device__ __forceinline__ void fft2_load_rows(typename FT<R>::C (&v)[8], const void *p, long long base, int d0, int t,
+                                               bool two) {
+    const T *a = (const T *)p + base, *b = a + (two ? d0 : 0);
+    T x[8], y[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        if (NT * j >= d0) break;  // the padding, for the whole workgroup
+        const int n = min(t + NT * j, d0 - 1);
+        x[j] = a[n];
+        y[j] = b[n];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const bool ok = t + NT * j < d0;
+        v[j].x = ok ? (R)x[j] : (R)0;
+        v[j].y = ok && two ? (R)y[j] : (R)0;
+    }
+}
+
+template <typename R, int NT>
+__device__ __forceinline__ void fft2_load_any(int type, typename FT<R>::C (&v)[8], const void *p, long long base,
+                                              int d0, int t, bool two) {
+    if constexpr (sizeof(R) == 8) {
+        fft2_load_rows<double, R, NT>(v, p, base, d0, t, two);
+    } else {
+        switch (type) {
+            case DT_F32: fft2_load_rows<float, R, NT>(v, p, base, d0, t, two); break;
+            case DT_S32: fft2_load_rows<int32_t, R, NT>(v, p, base, d0, t, two); break;
+            case DT_U32: fft2_load_rows<uint32_t, R, NT>(v, p, base, d0, t, two); break;
+            case DT_S16: fft2_load_rows<int16_t, R, NT>(v, p, base, d0, t, two); break;
+            case DT_U16: fft2_load_rows<uint16_t, R, NT>(v, p, base, d0, t, two); break;
+            case DT_S64: fft2_load_rows<long long, R, NT>(v, p, base, d0, t, two); break;
+            case DT_U64: fft2_load_rows<unsigned long long, R, NT>(v, p, base, d0, t, two); break;
+            case DT_U8: fft2_load_rows<uint8_t, R, NT>(v, p, base, d0, t, two); break;
+            default: fft2_load_rows<int8_t, R, NT>(v, p, base, d0, t, two); break;  // s8, b8
+        }
+    }
+}
+
+// Eight points of a column of n0 rows, zeros past them.
+template <typename R, int NT>
+__device__ __forceinline__ void fft2_load_col(typename FT<R>::C (&v)[8], const typename FT<R>::C *c, int n0, int t) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        if (NT * j >= n0) break;  // the padding, for the whole workgroup
+        v[j] = c[min(t + NT * j, n0 - 1)];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        if (t + NT * j >= n0) v[j] = FT<R>::mk(0, 0);
+}
+
+// Eight points each of two result rows; integers of the batched path round to
+// nearest.
+template <typename T, typename R, int NT>
+__device__ __forceinline__ void fft2_store_rows(const typename FT<R>::C (&v)[8], void *p, long long base, int off,
+                                                int o0, int t, bool two, R scale) {
+    T *a = (T *)p + base, *b = a + o0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int n = t + NT * j - off;
+        const R x = v[j].x * scale, y = v[j].y * scale;
+        if (n < 0 || n >= o0) continue;
+        if constexpr (std::is_floating_point<T>::value) {
+            a[n] = (T)x;
+            if (two) b[n] = (T)y;
+        } else {
+            a[n] = (T)roundf((float)x);
+            if (two) b[n] = (T)roundf((float)y);
+        }
+    }
+}
+
+template <typename R, int NT>
+__device__ __forceinline__ void fft2_store_any(int type, const typename FT<R>::C (&v)[8], void *p, long long base,
+                                               int off, int o0, int t, bool two, R scale) {
+    if constexpr (sizeof(R) == 8) {
+        fft2_store_rows<double, R, NT>(v, p, base, off, o0, t, two, scale);
+    } else {
+        switch (type) {
+            case DT_F32: fft2_store_rows<float, R, NT>(v, p, base, off, o0, t, two, scale); break;
+            case DT_S32: fft2_store_rows<int32_t, R, NT>(v, p, base, off, o0, t, two, scale); break;
+            case DT_U32: fft2_store_rows<uint32_t, R, NT>(v, p, base, off, o0, t, two, scale); break;
+            case DT_S16: fft2_store_rows<int16_t, R, NT>(v, p, base, off, o0, t, two, scale); break;
+            case DT_U16: fft2_store_rows<uint16_t, R, NT>(v, p, base, off, o0, t, two, scale); break;
+            case DT_S64: fft2_store_rows<long long, R, NT>(v, p, base, off, o0, t, two, scale); break;
+            case DT_U64: fft2_store_rows<unsigned long long, R, NT>(v, p, base, off, o0, t, two, scale); break;
+            case DT_U8: fft2_store_rows<uint8_t, R, NT>(v, p, base, off, o0, t, two, scale); break;
+            default: fft2_store_rows<int8_t, R, NT>(v, p, base, off, o0, t, two, scale); break;
+        }
+    }
+}
+
+// the spectra of two adjacent rows at one column: one 16- or 32-byte access
+template <typename R>
+struct alignas(4 * sizeof(R)) Fft2Pair {
+    R ax, ay, bx, by;
+};
+
+template <typename R, int LOGL>
+__global__ __launch_bounds__((RegFft<R, LOGL>::THREADS)) void fft2_rows(typename FT<R>::C *__restrict__ ws,
+                                                                        Fft2Side sg, Fft2Side fl) {
+    using F = RegFft<R, LOGL>;
+    using C = typename FT<R>::C;
+    __shared__ C buf[F::TPW * F::PITCH];
+    const int g = threadIdx.x / F::NT, t = threadIdx.x % F::NT;
+    C *lds = buf + g * F::PITCH;
+    F f;
+    f.init(t);
+    // neighbouring row pairs write parts of the same lines: keep them on one XCD
+    const unsigned u = (unsigned)xcd_remap(blockIdx.x, gridDim.x) * F::TPW + g;
+    const bool in_sig = u < sg.ntrans, live = u < sg.ntrans + fl.ntrans;
+    const Fft2Side &s = in_sig ? sg : fl;
+    const unsigned w = in_sig ? u : u - sg.ntrans;
+    const unsigned b = w / (unsigned)s.pairs;
+    const int r = 2 * (int)(w - b * (unsigned)s.pairs);
+    const long long base = ((long long)b * s.d1 + r) * s.d0;
+    const bool two = live && r + 1 < s.d1;
+    C v[8];
+    fft2_load_any<R, F::NT>(s.type, v, s.p, live ? base : 0, s.d0, t, two);
+    f.template run<false>(v, lds, t);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 8; ++j) lds[F::row(t) + j * F::ROW] = v[j];
+    __syncthreads();
+    if (!live) return;
+    Fft2Pair<R> *o = (Fft2Pair<R> *)(ws + s.out) + ((long long)b * (F::L / 2 + 1) * s.pitch + r) / 2;
+    for (int k = t; k <= F::L / 2; k += F::NT) {
+        const C z = lds[F::at(k)], n = lds[F::at((F::L - k) & (F::L - 1))];
+        Fft2Pair<R> q;  // A = (z + conj n) / 2, B = (z - conj n) / 2i
+        q.ax = (R)0.5 * (z.x + n.x);
+        q.ay = (R)0.5 * (z.y - n.y);
+        q.bx = (R)0.5 * (z.y + n.y);
+        q.by = (R)0.5 * (n.x - z.x);
+        o[(long long)k * (s.pitch / 2)] = q;
+    }
+}
+
+struct Fft2Cols {
+    long long a, b, o;        // spectra of operand A and B, result (element offsets)
+    int ra, rb, ro;           // their rows
+    int pa, pb, po;           // their pitches
+    int H, off;               // columns per slice, first row of the result
+    int asl, bsl;             // 1: A / B has a slice per result slice, 0: one for all
+    int nob, per;             // result slices, slices per workgroup row
+};
+
+// Result slice i = A[i * asl] x B[i * bsl]; A's spectrum is transformed once
+// where one slice serves all.
+template <typename R, int LOGL>
+__global__ __launch_bounds__((RegFft<R, LOGL>::THREADS)) void fft2_cols(typename FT<R>::C *ws, Fft2Cols p) {
+    using F = RegFft<R, LOGL>;
+    using C = typename FT<R>::C;
+    __shared__ C buf[F::TPW * F::PITCH];
+    const int g = threadIdx.x / F::NT, t = threadIdx.x % F::NT;
+    C *lds = buf + g * F::PITCH;
+    F f;
+    f.init(t);
+    const int k0 = blockIdx.x * F::TPW + g;
+    const bool live = k0 < p.H;
+    const int kc = live ? k0 : p.H - 1;
+    C a[8];
+    for (int i = blockIdx.y * p.per; i < min((int)(blockIdx.y + 1) * p.per, p.nob); ++i) {
+        C v[8];
+        fft2_load_col<R, F::NT>(v, ws + p.b + ((long long)(i * p.bsl) * p.H + kc) * p.pb, p.rb, t);
+        if (p.asl || i == (int)blockIdx.y * p.per) {
+            fft2_load_col<R, F::NT>(a, ws + p.a + ((long long)(i * p.asl) * p.H + kc) * p.pa, p.ra, t);
+            f.template run<false>(a, lds, t);
+        }
+        f.template run<false>(v, lds, t);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = cmul2(v[j], a[j]);
+        f.template run<true>(v, lds, t);
+        C *vo = ws + p.o + ((long long)i * p.H + k0) * p.po - p.off;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int n = t + F::NT * j;
+            if (live && n >= p.off && n < p.off + p.ro) vo[n] = v[j];
+        }
+    }
+}
+
+struct Fft2Out {
+    void *p;
+    long long in;        // spectrum offset
+    int type, o0, o1;    // output slice
+    int pairs, pitch, off;
+    unsigned ntrans;
+};
+
+template <typename R, int LOGL>
+__global__ __launch_bounds__((RegFft<R, LOGL>::THREADS)) void fft2_rows_inv(const typename FT<R>::C *__restrict__ ws,
+                                                                            Fft2Out s, R scale) {
+    using F = RegFft<R, LOGL>;
+    using C = typename FT<R>::C;
+    __shared__ C buf[F::TPW * F::PITCH];
+    const int g = threadIdx.x / F::NT, t = threadIdx.x % F::NT;
+    C *lds = buf + g * F::PITCH;
+    F f;
+    f.init(t);
+    const unsigned u = (unsigned)xcd_remap(blockIdx.x, gridDim.x) * F::TPW + g;
+    const bool live = u < s.ntrans;
+    const unsigned b = u / (unsigned)s.pairs;
+    const int r = 2 * (int)(u - b * (unsigned)s.pairs);
+    const bool two = r + 1 < s.o1;
+    C v[8];
+    const Fft2Pair<R> *q = (const Fft2Pair<R> *)(ws + s.in) +
+                           (live ? ((long long)b * (F::L / 2 + 1) * s.pitch + r) / 2 : 0);
+    Fft2Pair<R> z[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) z[j] = q[(long long)min(t + F::NT * j, F::L / 2) * (s.pitch / 2)];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+        const int k = t + F::NT * j;
+        if (!two) z[j].bx = z[j].by = 0;
+        if (k == 0 || k == F::L / 2) {
+            // real rows have real spectra there
+            lds[F::at(k)] = FT<R>::mk(z[j].ax, z[j].bx);
+        } else if (k < F::L / 2) {
+            lds[F::at(k)] = FT<R>::mk(z[j].ax - z[j].by, z[j].ay + z[j].bx);
+            lds[F::at(F::L - k)] = FT<R>::mk(z[j].ax + z[j].by, z[j].bx - z[j].ay);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = lds[F::row(t) + j * F::ROW];
+    f.template run<true>(v, lds, t);
+    if (!live) return;
+    fft2_store_any<R, F::NT>(s.type, v, s.p, ((long long)b * s.o1 + r) * s.o0, s.off, s.o0, t, two, scale);
+}
+
 // ---------------------------------------------------------------- host side
 static long long nextpow2ll(long long x) {
     long long p = 1;
@@ -302,7 +544,7 @@ static int ensure_twiddles(hipStream_t s) {
     if (!g_tw_ready[dev]) {
         // filled once per device; the wait makes the table visible to work
         // queued later on any stream of the device
-        fft_twiddle_init<<<8, 256, 0, s>>>();
+        fft_twiddle_init<<<32, 256, 0, s>>>();
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) return K_ERR_RUNTIME;
         g_tw_ready[dev] = true;
     }
@@ -448,6 +690,112 @@ static int crop_any(int type, void *out, const void *O, const long long *od, con
     return launch_status();
 }
 
+// ------------------------------------------- host side, two-dimensional
+// Real data of one precision whose padded sides are 64..4096 (one transform in
+// at most 64 KB of LDS, at most eight transforms per wave); anything else
+// runs the general passes (1024^2 f32: 33 us here, 474 us there).
+static bool fft2_serves(int dtype, int ftype, const long long *sd, const long long *fd, const long long *od, int kind,
+                        int rank, const FftPlan &P) {
+    if (rank != 2 || kind < 1 || kind > 4 || ftype != dtype || is_complex(dtype)) return false;
+    const long long lmax = P.dbl ? 2048 : 4096;
+    for (int k = 0; k < 2; ++k)
+        if (sd[k] < 1 || fd[k] < 1 || P.L[k] < 64 || P.L[k] > lmax) return false;
+    const long long lim = 1LL << 30;  // transforms and slices are counted in 32 bits
+    const long long rs = (sd[1] + 1) / 2 * P.nbs, rf = (fd[1] + 1) / 2 * P.nbf, ro = (od[1] + 1) / 2 * P.nbo;
+    return rs < lim && rf < lim && ro < lim && P.nbo < lim;
+}
+
+// runs LOGL = 6..12 (6..11 for double)
+template <typename R, typename Fn>
+static void fft2_by_length(long long L, Fn fn) {
+    switch (L) {
+        case 64: fn(std::integral_constant<int, 6>()); break;
+        case 128: fn(std::integral_constant<int, 7>()); break;
+        case 256: fn(std::integral_constant<int, 8>()); break;
+        case 512: fn(std::integral_constant<int, 9>()); break;
+        case 1024: fn(std::integral_constant<int, 10>()); break;
+        case 2048: fn(std::integral_constant<int, 11>()); break;
+        default:
+            if constexpr (sizeof(R) == 4) fn(std::integral_constant<int, 12>());
+    }
+}
+
+// Spectrum rows per column: whole 16-value groups and an odd number of them,
+// so that columns start on their own cache lines and equal rows of adjacent
+// columns spread over the L2 channels (a pitch of 1024 values puts them all
+// into one).
+static int fft2_pitch(long long rows) { return (int)(((rows + 15) / 16 | 1) * 16); }
+
+template <typename R>
+static int fft2_run(int dtype, void *out, const long long *od, const void *in, const long long *sd, const void *filt,
+                    const long long *fd, int kind, bool expand, char *ws, const FftPlan &P, hipStream_t s) {
+    using C = typename FT<R>::C;
+    const int H = (int)(P.L[0] / 2 + 1);
+    const bool rhs = kind == 3;
+    Fft2Side sg{}, fl{};
+    auto side = [&](Fft2Side &x, const void *p, const long long *d, long long nb, long long res) {
+        x.p = p;
+        x.type = dtype;
+        x.d0 = (int)d[0];
+        x.d1 = (int)d[1];
+        x.pairs = (int)((d[1] + 1) / 2);
+        // the result takes the place of the operand it has a slice for
+        x.pitch = fft2_pitch(d[1] > res ? d[1] : res);
+        x.ntrans = (unsigned)(x.pairs * nb);
+    };
+    side(sg, in, sd, P.nbs, rhs ? 0 : od[1]);
+    side(fl, filt, fd, P.nbf, rhs ? od[1] : 0);
+    fl.out = (long long)H * sg.pitch * P.nbs;
+    C *w = (C *)ws;
+    fft2_by_length<R>(P.L[0], [&](auto lg) {
+        using F = RegFft<R, decltype(lg)::value>;
+        const unsigned blocks = (sg.ntrans + fl.ntrans + F::TPW - 1) / F::TPW;
+        fft2_rows<R, decltype(lg)::value><<<blocks, F::THREADS, 0, s>>>(w, sg, fl);
+    });
+    // A: the operand with one slice for all (NONE and LHS: the filter)
+    const Fft2Side &a = rhs ? sg : fl, &b = rhs ? fl : sg;
+    Fft2Cols c{};
+    c.a = a.out;
+    c.b = b.out;
+    c.o = b.out;
+    c.ra = a.d1;
+    c.rb = b.d1;
+    c.ro = (int)od[1];
+    c.pa = a.pitch;
+    c.pb = c.po = b.pitch;
+    c.H = H;
+    c.off = expand ? 0 : (int)(fd[1] / 2);
+    c.asl = kind == 4 ? 1 : 0;
+    c.bsl = 1;
+    c.nob = (int)P.nbo;
+    fft2_by_length<R>(P.L[1], [&](auto lg) {
+        using F = RegFft<R, decltype(lg)::value>;
+        const int gx = (H + F::TPW - 1) / F::TPW;
+        // about eight workgroups per CU; more slices than that share A's transform
+        const long long want = (2048 + gx - 1) / gx;
+        c.per = (int)((P.nbo + want - 1) / want);
+        const unsigned gy = (unsigned)((P.nbo + c.per - 1) / c.per);
+        fft2_cols<R, decltype(lg)::value><<<dim3(gx, gy), F::THREADS, 0, s>>>(w, c);
+    });
+    Fft2Out o{};
+    o.p = out;
+    o.in = b.out;
+    o.type = dtype;
+    o.o0 = (int)od[0];
+    o.o1 = (int)od[1];
+    o.pairs = (int)((od[1] + 1) / 2);
+    o.pitch = b.pitch;
+    o.off = expand ? 0 : (int)(fd[0] / 2);
+    o.ntrans = (unsigned)(o.pairs * P.nbo);
+    const R scale = (R)1 / (R)P.PS;  // a power of two
+    fft2_by_length<R>(P.L[0], [&](auto lg) {
+        using F = RegFft<R, decltype(lg)::value>;
+        const unsigned blocks = (o.ntrans + F::TPW - 1) / F::TPW;
+        fft2_rows_inv<R, decltype(lg)::value><<<blocks, F::THREADS, 0, s>>>(w, o, scale);
+    });
+    return launch_status();
+}
+
 template <typename R>
 static int fft_convolve_run(int dtype, void *out, const long long *od, const void *in, const long long *sd,
                             int ftype, const void *filt, const long long *fd, int kind, int rank, bool expand,
@@ -459,6 +807,8 @@ static int fft_convolve_run(int dtype, void *out, const long long *od, const voi
     C *O = diff ? F + P.PS * P.nbf : (kind == 3 ? F : S);  // RHS: in place in F; DIFF: its own buffer
     int rc = ensure_twiddles(s);
     if (rc) return rc;
+    if (fft2_serves(dtype, ftype, sd, fd, od, kind, rank, P))
+        return fft2_run<R>(dtype, out, od, in, sd, filt, fd, kind, expand, ws, P, s);
     if ((rc = pad_any<R>(dtype, S, in, sd, P, rank, P.nbs, s))) return rc;
     if ((rc = pad_any<R>(ftype, F, filt, fd, P, rank, P.nbf, s))) return rc;
     long long st = 1;
