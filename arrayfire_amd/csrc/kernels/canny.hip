@@ -18,9 +18,12 @@
 //    through the 8 linear-offset neighbours; the marked set is the closure of
 //    the seeds over weak pixels, computed here by repeated sweeps that mark a
 //    weak pixel next to a marked one, until a sweep changes nothing.
+// af_canny itself runs the tile kernels of canny_tiles.hip (and canny_otsu);
+// the kernels here are the steps one by one, for callers of the kernel ABI.
 // Arithmetic is uncontracted and in the reference's order, so every
 // comparison sees the reference's values.
 #include "kcommon.hpp"
+#include "../canny.hpp"
 #include "../../../include/afhip_kernels.h"
 
 namespace afhip {
@@ -283,6 +286,11 @@ __global__ __launch_bounds__(256) void canny_sweep(unsigned char *__restrict__ o
         }
     }
     if (ch) changed[0] = 1;
+}
+
+int canny_otsu_lanes(float *thr, const unsigned *hist, long long per, long long ns, int nbins, hipStream_t s) {
+    canny_otsu<<<(unsigned)((ns + 63) / 64), 64, 0, s>>>(thr, hist, nbins, ns, (float)per);
+    return launch_status();
 }
 
 }  // namespace afhip
