@@ -212,13 +212,12 @@ static int device_cus() {
     return n;
 }
 
-// ---- NN variant choice. Layers whose patch kernels would leave most CUs
-// idle, and every layer the patch kernels do not serve, run the gather GEMM
-// with a split reduction; the autotuner (autotune.cpp) times the candidate
-// variants (the patch kernels where they serve; split counts 1, 2, 4, 8, 16)
-// on the first call of a geometry and caches the fastest under a key of
-// (pass, dtypes, precision, dims, stride, padding, dilation). Under stream
-// capture only cached choices are used. AFHIP_NN_AUTOTUNE=0 (or an explicit
+// ---- NN variant choice. The autotuner (autotune.cpp) times the candidate
+// variants (the patch kernels or the polyphase split where they serve; the
+// GEMM, with splits of the reduction where its tiles leave CUs idle) on the
+// first call of a geometry and caches the fastest under a key of (pass,
+// dtypes, precision, dims, stride, padding, dilation). Under stream capture
+// only cached choices are used. AFHIP_NN_AUTOTUNE=0 (or an explicit
 // AFHIP_NN_SPLIT) keeps the built-in rules.
 static bool nn_autotune_on() {
     const char *a = std::getenv("AFHIP_NN_AUTOTUNE");
@@ -285,22 +284,28 @@ static void run_patch_kernels(int pass, const ArrayImpl &in, const ArrayImpl &w,
             pass == 0 ? "convolve2_nn" : "convolve2_gradient_nn");
 }
 
-// Candidate list: [patch kernels (when they serve)] + gather GEMM splits.
+// Candidates: `first` (the patch kernels or the polyphase split, where they
+// serve), then the GEMM with the split counts worth a try. Splitting pays
+// only where the GEMM's own tiles leave CUs idle.
 static std::vector<std::function<void()>> nn_candidates(int pass, const ArrayImpl &in, const ArrayImpl &w,
                                                         af_dtype out_type, int precision, void *out,
-                                                        const NNGeom &g, long long patch_need) {
+                                                        const NNGeom &g, std::function<void()> first) {
     std::vector<std::function<void()>> c;
-    if (patch_need > 0)
-        c.push_back([=, &in, &w, &g] { run_patch_kernels(pass, in, w, out_type, precision, out, g, patch_need); });
+    if (first) c.push_back(std::move(first));
+    const dim4 &o = pass == 0 ? g.y : g.x;
+    const long long tiles = (o[2] + 127) / 128 * ((o[0] * o[1] * o[3] + 127) / 128);
     for (int sp : kSplitCands)
-        c.push_back([=, &in, &w, &g] { run_gemm_split(pass, in, w, out_type, precision, out, g, sp); });
+        if (sp == 1 || tiles < device_cus())
+            c.push_back([=, &in, &w, &g] { run_gemm_split(pass, in, w, out_type, precision, out, g, sp); });
     return c;
 }
 
-// The patch kernels for layers that fill the chip with them; otherwise the
-// autotuned choice between them and the split gather GEMM (built-in rule:
-// the GEMM when the patch kernels launch fewer workgroups than a quarter of
-// the CUs). AFHIP_NN_SMALL=0 keeps every served layer on the patch kernels.
+// The autotuned choice between the patch kernels and the GEMM: neither wins by
+// a rule that the shape alone gives (BF16 56x56x64x32 -> 128: 28 us on the
+// weights-resident kernel, 42 us on the GEMM; 28x28x128x32 -> 128, whose rows
+// are no whole 16-byte vectors: 55 and 24; 79x79x3x32 -> 32: 34 and 43).
+// Built-in rule: the patch kernels when they launch at least a quarter of the
+// CUs' workgroups. AFHIP_NN_SMALL=0 keeps every served layer on them.
 static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype out_type,
                       int precision, void *out, const NNGeom &g) {
     const char *env = std::getenv("AFHIP_NN_GATHER");
@@ -308,17 +313,19 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
     const long long need = afhip_k_conv2_nn_patch_workspace(pass, in.type, precision, g.x.d, g.w.d,
                                                             g.y.d, g.st, g.pd, g.dl);
     if (need <= 0) return false;
+    auto patch = [=, &in, &w, &g] { run_patch_kernels(pass, in, w, out_type, precision, out, g, need); };
     const char *sm = std::getenv("AFHIP_NN_SMALL");
-    const long long tiles = afhip_k_conv2_nn_patch_tiles(pass, in.type, precision, g.x.d, g.w.d, g.y.d, g.st,
-                                                         g.pd, g.dl);
-    const int cus = device_cus();
-    if ((sm && sm[0] == '0') || tiles >= cus) {
-        run_patch_kernels(pass, in, w, out_type, precision, out, g, need);
+    if (sm && sm[0] == '0') {
+        patch();
         return true;
     }
-    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, need);
-    int c = nn_pick(nn_key("nn", pass, in, out_type, precision, g), cands);
-    if (c < 0) c = (tiles > 0 && tiles * 4 >= cus) ? 0 : -1;  // the rule
+    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, patch);
+    int c = nn_pick(nn_key("nn2", pass, in, out_type, precision, g), cands);
+    if (c < 0) {
+        const long long tiles = afhip_k_conv2_nn_patch_tiles(pass, in.type, precision, g.x.d, g.w.d, g.y.d, g.st,
+                                                             g.pd, g.dl);
+        c = tiles * 4 >= device_cus() ? 0 : -1;
+    }
     if (c >= 0)
         cands[c]();
     else
@@ -326,12 +333,15 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
     return true;
 }
 
-// The gather GEMM for every geometry, its split count autotuned (built-in
-// rule: split when that fills the chip).
+// The GEMM for every other geometry, its split count autotuned (built-in
+// rule: split when that fills the chip); `first`: another kernel that serves,
+// the built-in choice when the autotuner is off.
 static void run_gemm(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype out_type, int precision,
-                     void *out, const NNGeom &g) {
-    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, 0);
-    const int c = nn_pick(nn_key("nn_gemm", pass, in, out_type, precision, g), cands);
+                     void *out, const NNGeom &g, std::function<void()> first = nullptr) {
+    const bool has_first = (bool)first;
+    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, std::move(first));
+    int c = nn_pick(nn_key("nn_gemm2", pass, in, out_type, precision, g), cands);
+    if (c < 0 && has_first) c = 0;
     if (c >= 0)
         cands[c]();
     else
@@ -376,19 +386,21 @@ static af_array conv2_data_grad(const ArrayImpl &dy, const ArrayImpl &x, const A
         return out.release();
     }
     if (run_patch(1, dy, w, out_type, precision, o, g)) return out.release();
-    // strided layers: the polyphase split into stride-1 convolutions on the
-    // patch kernels when its phases fill the chip, else the split gather
-    // GEMM over phase-ordered pixels (AFHIP_NN_GATHER=1 keeps the gather
-    // kernel)
+    // strided layers: the autotuned choice between the polyphase split into
+    // stride-1 convolutions on the patch kernels, when its phases fill the
+    // chip, and the GEMM over phase-ordered pixels (AFHIP_NN_GATHER=1 keeps
+    // the GEMM)
     const char *gather = std::getenv("AFHIP_NN_GATHER");
     if (!(gather && gather[0] == '1')) {
         const long long pb = afhip_k_conv2_nn_dgrad_poly_workspace(x.type, out_type, precision, g.x.d, g.w.d,
                                                                   g.y.d, g.st, g.pd, g.dl);
         if (pb > 0) {
-            auto ws = scratch((size_t)pb);
-            check_k(afhip_k_conv2_nn_dgrad_poly(x.type, out_type, precision, o, dy.data(), w.data(), g.x.d, g.w.d,
-                                                g.y.d, g.st, g.pd, g.dl, ws->ptr, pb, stream()),
-                    "convolve2_gradient_nn");
+            run_gemm(1, dy, w, out_type, precision, o, g, [&] {
+                auto ws = scratch((size_t)pb);
+                check_k(afhip_k_conv2_nn_dgrad_poly(x.type, out_type, precision, o, dy.data(), w.data(), g.x.d,
+                                                    g.w.d, g.y.d, g.st, g.pd, g.dl, ws->ptr, pb, stream()),
+                        "convolve2_gradient_nn");
+            });
             return out.release();
         }
     }

@@ -30,6 +30,9 @@
 //   SPLIT hi = bf16(v), lo = bf16(v - hi); hi*hi' + hi*lo' + lo*hi' on BF16
 // Accumulation is FP32 in every mode. One LDS buffer; the next slice's global
 // loads are in flight in registers while the current slice is multiplied.
+// nn_gemm gathers its operands element by element and takes any geometry and
+// conversion; nn_clgemm (below) reads channel-last copies where the operands
+// are stored in the MMA type.
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -49,7 +52,7 @@ enum Pass : int { P_FWD = 0, P_DGRAD = 1, P_WGRAD = 2 };
 
 // Strided data gradients order their columns by stride phase when there are
 // at most this many phases (s0 * s1).
-constexpr int kMaxPhases = 16;
+constexpr int kMaxPhases = 256;
 
 struct NNParams {
     // x [W,H,C,N], w [fw,fh,C,K], y [OW,OH,K,N]
@@ -451,148 +454,393 @@ struct Gather<TIn, P_WGRAD> {
     }
 };
 
-// Slices of the channel-last path in flight per lane (register sets).
-constexpr int CL_DEPTH = 4;
+// ------------------------------------------------- channel-last GEMM
+// Operands stored in the MMA type run here. They are first copied channel-last: the weights
+// as Wp [RS][M][Rcp] (forward M = K, R = C, Wp[t][k][c] =
+// w[k][c][fh-1-j][fw-1-i]; data gradient M = C, R = K, Wp[t][c][k] = the same
+// element; t = j*fw + i) and the activation as [N][rows][cols][Rcp], zeros
+// past the reduction channels.
 
-// ---- channel-last gathers: each lane's 16 R values are one contiguous run
-// of 16 channels (2 or 4 aligned 16-byte loads) for A and for B.
-template <typename T, int PASS>
-struct GatherCL {
-    static constexpr int Q = (int)sizeof(T);  // 16-byte vectors per 16 values
-    const T *act, *wp;
-    const NNParams &p;
-    long long arow;
-    bool bvalid;
-    int bn, ba, bb;   // image; output row, column (forward) or input y, x (data gradient)
-    int rx, ry, Ti;   // phased data gradient: the tile's phase, its tap count along W
-    __device__ GatherCL(const T *act_, const T *wp_, const NNParams &p_, long long ar, long long br, int ph)
-        : act(act_), wp(wp_), p(p_), arow(ar) {
-        rx = ry = 0;
-        Ti = p.fw;
-        if (PASS == P_DGRAD && p.phased) {
-            rx = ph % p.s0;
-            ry = ph / p.s0;
-            const int Mx = phase_len(p.W, p.s0, rx), My = phase_len(p.H, p.s1, ry);
-            bvalid = br < (long long)p.N * My * Mx;
-            const Pix q = decode(bvalid ? br : 0, My, Mx);
-            bn = q.n;
-            ba = p.s1 * q.a + ry;
-            bb = p.s0 * q.b + rx;
-            Ti = phase_taps(p.fw, rx, p.p0, p.d0, p.s0);
-        } else {
-            bvalid = br < p.Ncol;
-            const Pix q = PASS == P_FWD ? decode(bvalid ? br : 0, p.OH, p.OW) : decode(bvalid ? br : 0, p.H, p.W);
-            bn = q.n;
-            ba = q.a;
-            bb = q.b;
-        }
-    }
-    // Buffer loads: an operand outside the image (or a row past M) reads
-    // zeros from an offset past the resource's end, so every lane issues the
-    // same loads and the prefetch ring's waits count them exactly.
-    __device__ void load(long long ks, int kk0, uint4 (&ra)[Q], uint4 (&rb)[Q]) const {
-        constexpr int kOOB = 0x7fffffc0;
-        const int u = (int)(ks / p.kchunks);
-        const int c0 = (int)(ks - (long long)u * p.kchunks) * BK + kk0;
-        int i, j;
-        if (PASS == P_DGRAD && p.phased) {
-            i = phase_tap_at(p.fw, rx, p.p0, p.d0, p.s0, u % Ti);
-            j = phase_tap_at(p.fh, ry, p.p1, p.d1, p.s1, u / Ti);
-        } else {
-            i = u % p.fw;
-            j = u / p.fw;
-        }
-        const int t = j * p.fw + i;
-        const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(wp), (short)0, p.wp_bytes, 0x00020000);
-        const auto ra_ = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(act), (short)0, p.act_bytes, 0x00020000);
-        const int offa = arow < p.M ? (int)((((long long)t * p.M + arow) * p.Rcp + c0) * (long long)sizeof(T)) : kOOB;
-        bool ok;
-        long long off;
-        if constexpr (PASS == P_FWD) {
-            const int ih = ba * p.s1 - p.p1 + j * p.d1;
-            const int iw = bb * p.s0 - p.p0 + i * p.d0;
-            ok = bvalid && ih >= 0 && ih < p.H && iw >= 0 && iw < p.W;
-            off = (((long long)bn * p.H + ih) * p.W + iw) * p.Rcp + c0;
-        } else {
-            const int nh = ba + p.p1 - j * p.d1;
-            const int nw = bb + p.p0 - i * p.d0;
-            ok = bvalid && nh >= 0 && nw >= 0 && (nh % p.s1) == 0 && (nw % p.s0) == 0;
-            const int oh = ok ? nh / p.s1 : 0, ow = ok ? nw / p.s0 : 0;
-            ok = ok && oh < p.OH && ow < p.OW;
-            off = (((long long)bn * p.OH + oh) * p.OW + ow) * p.Rcp + c0;
-        }
-        const int offb = ok ? (int)(off * (long long)sizeof(T)) : kOOB;
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            ra[q] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, offa + 16 * q, 0, 0));
-            rb[q] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra_, offb + 16 * q, 0, 0));
-        }
-    }
-};
-
-// Writes one lane's 16 raw values (row, R offset kk0) of an operand tile.
-template <int MODE>
-__device__ inline void store_raw16(char *tile, int row, int kk0, const uint4 *v) {
-    constexpr int P = Lds<MODE>::PITCH, E = Lds<MODE>::ESZ;
-    uint4 *t = reinterpret_cast<uint4 *>(tile + (row * P + kk0) * E);
-#pragma unroll
-    for (int q = 0; q < E; ++q) t[q] = v[q];
-}
-
-// Wp [RS][M][Rcp]: forward M = K, R = C, Wp[t][k][c] = w[k][c][fh-1-j][fw-1-i];
-// data gradient M = C, R = K, Wp[t][c][k] = the same element (t = j*fw + i).
-// Both channel-last copies in one launch: the first nbw workgroups pack the
-// weights into Wp (above), the others transpose the activation:
-// dst [N][rows][cols][Cp] <- src [N][Cd][rows][cols] (NCHW to channel-last),
-// zero for the channels past Cd, one lane writing 16 bytes of channels.
+// Both copies in one launch. The first nbw workgroups pack the weights, one
+// element per lane; each of the others transposes 64 pixels by 128 bytes of
+// channels through LDS, so that a wave reads 64 consecutive pixels of a
+// channel and writes whole 128-byte channel runs (an LDS row is 33 words: the
+// 64 pixels of a wave's write fall into 64 banks).
 template <typename T>
 __global__ __launch_bounds__(256) void nn_cl_copies(T *__restrict__ wp, const T *__restrict__ w, NNParams p,
                                                     int dgrad, int nbw, T *__restrict__ dst,
-                                                    const T *__restrict__ src, int cols, int rows, int Cd) {
+                                                    const T *__restrict__ src, int hw, int Cd, int npix, int ncg) {
     if ((int)blockIdx.x < nbw) {
-        const int Rc = dgrad ? p.K : p.C;
-        const long long total = (long long)p.RS * p.M * p.Rcp;
-        for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < total;
-             e += (long long)nbw * blockDim.x) {
-            const int r = (int)(e % p.Rcp);
-            const long long mt = e / p.Rcp;
-            const int m = (int)(mt % p.M);
-            const int t = (int)(mt / p.M);
-            const int i = t % p.fw, j = t / p.fw;
+        const int Rc = dgrad ? p.K : p.C, M = (int)p.M;
+        const unsigned total = (unsigned)(p.RS * M) * (unsigned)p.Rcp;  // below 2^31
+        for (unsigned e = blockIdx.x * 256u + threadIdx.x; e < total; e += (unsigned)nbw * 256u) {
+            const unsigned mt = e / (unsigned)p.Rcp;
+            const int r = (int)(e - mt * (unsigned)p.Rcp);
+            const int t = (int)(mt / (unsigned)M), m = (int)mt - t * M;
             T v{};
             if (r < Rc) {
                 const int k = dgrad ? r : m, c = dgrad ? m : r;
-                v = w[(((long long)k * p.C + c) * p.fh + (p.fh - 1 - j)) * p.fw + (p.fw - 1 - i)];
+                v = w[((long long)k * p.C + c) * p.RS + (p.RS - 1 - t)];
             }
             wp[e] = v;
         }
         return;
     }
-    constexpr int G = 16 / (int)sizeof(T);
-    const int Cp = p.Rcp, N = p.N;
-    const int cg = Cp / G;
-    const long long hw = (long long)rows * cols;
-    const long long total = (long long)N * hw * cg;
-    const long long nbt = (long long)gridDim.x - nbw;
-    for (long long e = (blockIdx.x - nbw) * (long long)blockDim.x + threadIdx.x; e < total;
-         e += nbt * blockDim.x) {
-        const int g = (int)(e % cg);
-        const long long pix = e / cg;  // n * hw + y * cols + x
-        const long long n = pix / hw, yx = pix - n * hw;
-        T v[G];
+    constexpr int CH = 128 / (int)sizeof(T);
+    __shared__ unsigned tile[64 * 33];
+    const unsigned b = blockIdx.x - nbw;
+    const int pb = (int)(b / (unsigned)ncg), c0 = (int)(b - (unsigned)pb * ncg) * CH;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int pix = pb * 64 + lane;
+    const int n = min(pix, npix - 1) / hw;
+    const T *s = src + (long long)n * Cd * hw + (min(pix, npix - 1) - n * hw);
+    T v[CH / 4];
 #pragma unroll
-        for (int q = 0; q < G; ++q) {
-            const int c = g * G + q;
-            v[q] = c < Cd ? src[(n * Cd + c) * hw + yx] : T{};
+    for (int u = 0; u < CH / 4; ++u) {
+        const int c = c0 + wave * (CH / 4) + u;
+        v[u] = s[(long long)min(c, Cd - 1) * hw];
+    }
+    T *row = reinterpret_cast<T *>(tile + lane * 33) + wave * (CH / 4);
+#pragma unroll
+    for (int u = 0; u < CH / 4; ++u) row[u] = c0 + wave * (CH / 4) + u < Cd ? v[u] : T{};
+    __syncthreads();
+    // 64 pixels x 8 groups of 16 bytes
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int e = (int)threadIdx.x + 256 * u, px = e >> 3, g = e & 7;
+        const int ch = c0 + g * (16 / (int)sizeof(T));
+        if (pb * 64 + px < npix && ch < p.Rcp) {
+            const unsigned *q = tile + px * 33 + g * 4;
+            *reinterpret_cast<uint4 *>(dst + (long long)(pb * 64 + px) * p.Rcp + ch) = make_uint4(q[0], q[1], q[2], q[3]);
         }
-        uint4 o;
-        __builtin_memcpy(&o, v, 16);
-        *reinterpret_cast<uint4 *>(dst + pix * Cp + g * G) = o;
+    }
+}
+
+// The taps a tile visits, as shifts of its pixels in the activation: tap (i, j)
+// of the walk reads column X + sx0 + i*dsx of row Y + sy0 + j*dsy and holds
+// filter tap t = (j0 + j*js)*fw + i0 + i*is. Forward: every tap, X = ow*s0.
+// Data gradient: the taps that reach the tile's stride phase, in the phase's
+// own pixel grid (all of them at stride 1).
+struct TapAxis {
+    int n, start, step, i0, is;
+};
+__device__ inline TapAxis tap_axis(bool fwd, bool phased, int f, int pd, int d, int s, int r) {
+    TapAxis a;
+    if (fwd || !phased) {
+        a.n = f;
+        a.i0 = 0;
+        a.is = 1;
+        a.start = fwd ? -pd : pd;
+        a.step = fwd ? d : -d;
+        return a;
+    }
+    // residues i with (r + pd - i*d) divisible by s: an arithmetic progression
+    a.n = a.i0 = 0;
+    a.is = 1;
+    int first = -1, second = -1;
+    for (int i = 0; i < f; ++i)
+        if (phase_tap(r, pd, i, d, s)) {
+            if (first < 0) first = i;
+            else if (second < 0) second = i;
+            ++a.n;
+        }
+    if (a.n) a.i0 = first;
+    if (a.n > 1) a.is = second - first;
+    a.start = (r + pd - a.i0 * d) / s;
+    a.step = -(a.is * d) / s;
+    return a;
+}
+
+// Output tile TM x TN per 256-lane workgroup, 2 x 2 waves. R is walked in
+// stages of 128 bytes per row: two 32-deep slices of 16-bit operands, one of
+// FP32, in the slice order of nn_gemm, so both give the same bits. LDS rows
+// are 128 bytes with their eight 16-byte groups XORed by the row, which keeps
+// the fragments' 16-byte reads free of bank conflicts without padding.
+// DEPTH register sets and two LDS buffers: a stage's loads are issued DEPTH
+// stages ahead and stored one stage ahead, with one barrier per stage. Every
+// lane follows the walk over (tap, channel slice) with counters of its own;
+// pixels outside the activation read zeros past the end of the buffer resource.
+// What bounds small layers is the latency of each stage's loads (the copies
+// were just written by other XCDs and come from the Infinity Cache, about a
+// microsecond away), which the depth covers, and the walk's address arithmetic
+// (about 50 instructions per stage beside 8 to 32 MFMAs). Copies included:
+// 27x27x96x16 -> 128, 5x5, F16 29 us (40 us before, of which 9 to sum splits);
+// 28x28x128x16 -> 128, 3x3, stride 2, BF16 15 us (25); its data gradient 19 us
+// (38); 75x70x128x8 -> 256, 3x3, BF16 58 us, 425 TFLOP/s (90 us on conv_patch).
+// Two stages of 256 bytes per row in place of four of 128 were no faster on
+// small layers (33 us for the 5x5) and slower on large ones (84 us).
+template <int MODE, typename T, typename TOut, int PASS, int TM, int TN>
+__global__ __launch_bounds__(NT, 2) void nn_clgemm(TOut *__restrict__ out, const T *__restrict__ act,
+                                                   const T *__restrict__ wp, float *__restrict__ partial,
+                                                   NNParams p) {
+    constexpr int SB = 128, DEPTH = TM + TN > 192 ? 2 : 4;
+    constexpr int E = (int)sizeof(T), CPS = SB / (32 * E);  // 32-deep slices per stage
+    constexpr int G = SB / 16, GPC = G / CPS;               // 16-byte groups per row, per slice
+    constexpr int RP = NT / G;                              // rows per load of the workgroup
+    constexpr int NA = TM / RP, NB = TN / RP;               // loads per lane and stage
+    constexpr int MI = TM / 32, NJ = TN / 32;               // 16 x 16 results per wave
+    __shared__ __attribute__((aligned(16))) char lds[2][(TM + TN) * SB];
+
+    const unsigned tiles = (unsigned)(p.tilesM * p.tilesN);
+    const unsigned bid = blockIdx.x;
+    const int split = (int)(bid / tiles);
+    const unsigned tl = bid - split * tiles;
+    const int tm = (int)(tl / (unsigned)p.tilesN), tn = (int)(tl - tm * (unsigned)p.tilesN);
+    const int m0 = tm * TM;
+    const bool phased = PASS == P_DGRAD && p.phased;
+    int ph = 0, n0 = tn * TN;
+    int rx = 0, ry = 0, gw, gh;  // the tile's pixel grid
+    if (phased) {  // phases start on whole tiles of BN columns
+        while (ph + 1 < p.nph && n0 >= p.ph_tile0[ph + 1] * BN) ++ph;
+        n0 -= p.ph_tile0[ph] * BN;
+        rx = ph % p.s0;
+        ry = ph / p.s0;
+        gw = phase_len(p.W, p.s0, rx);
+        gh = phase_len(p.H, p.s1, ry);
+    } else {
+        gw = PASS == P_FWD ? p.OW : p.W;
+        gh = PASS == P_FWD ? p.OH : p.H;
+    }
+    const TapAxis ax = tap_axis(PASS == P_FWD, phased, p.fw, p.p0, p.d0, p.s0, rx);
+    const TapAxis ay = tap_axis(PASS == P_FWD, phased, p.fh, p.p1, p.d1, p.s1, ry);
+    const int slices = ax.n * ay.n * p.kchunks;
+    const int kps = phased ? (slices + p.nsplit - 1) / p.nsplit : (int)p.ksteps_per_split;
+    const int q0 = split * kps, q1 = min(q0 + kps, slices);
+    const int cols = PASS == P_FWD ? p.W : p.OW, rows = PASS == P_FWD ? p.H : p.OH;
+    const int ncol = p.N * gw * gh;  // columns of the grid
+    if (n0 >= ncol) return;          // a phase's padding
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int grp = tid & (G - 1), lrow = tid / G;
+    const int pixb = p.Rcp * E;                    // bytes of a pixel's channels
+
+    int pX[NB], pY[NB], pBase[NB];
+#pragma unroll
+    for (int r = 0; r < NB; ++r) {
+        const int q = n0 + r * RP + lrow;
+        const unsigned qc = (unsigned)min(q, ncol - 1);
+        const int n = (int)(qc / (unsigned)(gw * gh));
+        const unsigned yx = qc - (unsigned)n * (gw * gh);
+        const int y = (int)(yx / (unsigned)gw), x = (int)yx - y * gw;
+        pX[r] = PASS == P_FWD ? x * p.s0 : x;
+        pY[r] = q < ncol ? (PASS == P_FWD ? y * p.s1 : y) : -(1 << 30);
+        pBase[r] = (int)(((unsigned)(n * rows + (PASS == P_FWD ? y * p.s1 : y)) * cols + pX[r]) * pixb);
+    }
+
+    // the lane's slice of the next stage to load: index, channel slice, tap
+    int q, c, ti, tj;
+    {
+        q = q0 + grp / GPC;
+        const int u = q / p.kchunks;
+        c = q - u * p.kchunks;
+        tj = ax.n > 0 ? u / ax.n : 0;
+        ti = u - tj * ax.n;
+    }
+    // one stage on: CPS slices are dt taps and dc slices (dt: dj rows of taps and di)
+    const int dt = CPS / p.kchunks, dc = CPS - dt * p.kchunks;
+    const int dj = ax.n > 0 ? dt / ax.n : 0, di = dt - dj * ax.n;
+    auto next = [&] {
+        q += CPS;
+        c += dc;
+        ti += di;
+        tj += dj;
+        if (c >= p.kchunks) {
+            c -= p.kchunks;
+            ++ti;
+        }
+        if (ti >= ax.n) {
+            ti -= ax.n;
+            ++tj;
+        }
+    };
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(wp), (short)0, p.wp_bytes, 0x00020000);
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(act), (short)0, p.act_bytes, 0x00020000);
+    struct Stage {
+        uint4 a[NA], b[NB];
+    };
+    auto load = [&](Stage &s) {
+        // Past the range the sign bit takes every offset out of the resource.
+        // The mask is opaque to the compiler: as a condition it became a branch
+        // around each load, with a wait for all loads in flight inside.
+        unsigned past = q < q1 ? 0u : 0x80000000u;
+        asm volatile("" : "+v"(past));
+        const int cb = c * (32 * E) + (grp % GPC) * 16;
+        const int t = (ay.i0 + tj * ay.is) * p.fw + ax.i0 + ti * ax.is;
+        const int sx = ax.start + ti * ax.step, sy = ay.start + tj * ay.step;
+        const unsigned woff = (unsigned)(t * (int)p.M + m0 + lrow) * (unsigned)pixb + cb;
+#pragma unroll
+        for (int r = 0; r < NA; ++r) {
+            const unsigned off = (woff + (unsigned)(RP * r * pixb)) | past | (m0 + lrow + RP * r < (int)p.M ? 0u : 0x80000000u);
+            s.a[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)off, 0, 0));
+        }
+        const unsigned soff = (unsigned)((sy * cols + sx) * pixb + cb);
+#pragma unroll
+        for (int r = 0; r < NB; ++r) {
+            const bool in = (unsigned)(pX[r] + sx) < (unsigned)cols && (unsigned)(pY[r] + sy) < (unsigned)rows;
+            unsigned off = (unsigned)pBase[r] + soff;
+            off = in ? off : 0x80000000u;
+            s.b[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(off | past), 0, 0));
+        }
+        next();
+    };
+    // the rows of a lane's loads agree in the bits that swizzle them
+    const int slot = lrow * SB + ((grp ^ (lrow & (G - 1))) * 16);
+    auto store = [&](const Stage &s, char *buf) {
+#pragma unroll
+        for (int r = 0; r < NA; ++r) *reinterpret_cast<uint4 *>(buf + slot + r * (RP * SB)) = s.a[r];
+#pragma unroll
+        for (int r = 0; r < NB; ++r) *reinterpret_cast<uint4 *>(buf + TM * SB + slot + r * (RP * SB)) = s.b[r];
+    };
+    const int wm = wave >> 1, wn = wave & 1;
+    const int r16 = lane & 15, g4 = lane >> 4;
+    f32x4_t acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const char *fa0 = lds[0] + (wm * (TM / 2) + r16) * SB, *fb0 = lds[0] + (TM + wn * (TN / 2) + r16) * SB;
+    // The operands are (pixels, weights): a lane's four results are four
+    // consecutive pixels of one output channel.
+    auto compute = [&](int buf) {
+        const char *fa = fa0 + buf * (int)sizeof(lds[0]), *fb = fb0 + buf * (int)sizeof(lds[0]);
+#pragma unroll
+        for (int h = 0; h < SB / 64; ++h) {
+            const int sw = ((4 * h + g4) ^ (r16 & (G - 1))) * 16;
+            uint4 a[MI], b[NJ];
+#pragma unroll
+            for (int i = 0; i < MI; ++i) a[i] = *reinterpret_cast<const uint4 *>(fa + i * (16 * SB) + sw);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) b[j] = *reinterpret_cast<const uint4 *>(fb + j * (16 * SB) + sw);
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    if constexpr (MODE == M_F32) {
+                        const float4 x = __builtin_bit_cast(float4, b[j]), y = __builtin_bit_cast(float4, a[i]);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, y.x, acc[i][j], 0, 0, 0);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, y.y, acc[i][j], 0, 0, 0);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, y.z, acc[i][j], 0, 0, 0);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, y.w, acc[i][j], 0, 0, 0);
+                    } else if constexpr (MODE == M_BF16) {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b[j]),
+                                                                            __builtin_bit_cast(bf16x8_t, a[i]),
+                                                                            acc[i][j], 0, 0, 0);
+                    } else {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, b[j]),
+                                                                           __builtin_bit_cast(f16x8_t, a[i]),
+                                                                           acc[i][j], 0, 0, 0);
+                    }
+                }
+        }
+    };
+
+    const int stages = q1 > q0 ? (q1 - q0 + CPS - 1) / CPS : 0;  // the same for every lane
+    if (stages > 0) {
+        // loads past the last stage read zeros and are never multiplied
+        Stage st[DEPTH];
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            load(st[d]);
+            // the loads stay in stage order: the loop's waits count them
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        store(st[0], lds[0]);
+        load(st[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        for (int k = 0;;) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) {
+                // stage k is in buffer d & 1; the other one was last read in
+                // stage k - 1, before this barrier
+                __syncthreads();
+                store(st[(d + 1) % DEPTH], lds[(d + 1) & 1]);
+                load(st[(d + 1) % DEPTH]);
+                compute(d & 1);
+                // straight out: an exit through the loop's end would make its
+                // first waits count the loads of this stage as the newest
+                if (++k == stages) goto done;
+            }
+        }
+    }
+done:
+
+    // acc[i][j][v]: channel m0 + wm*TM/2 + i*16 + r16, column n0 + wn*TN/2 + j*16 + 4*g4 + v
+    const int mlane = m0 + wm * (TM / 2) + r16;
+    if (p.nsplit > 1) {
+        const int pc0 = phased ? p.ph_tile0[ph] * BN : 0, nall = (int)p.Ncol;
+        float *pt = partial + (long long)split * p.M * p.Ncol;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int col = pc0 + n0 + wn * (TN / 2) + j * 16 + 4 * g4;
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                const int m = mlane + 16 * i;
+                if (m >= (int)p.M) continue;
+                float *o = pt + (long long)m * nall + col;
+                if ((nall & 3) == 0 && col + 4 <= nall) {
+                    *reinterpret_cast<float4 *>(o) = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (col + v < nall) o[v] = acc[i][j][v];
+                }
+            }
+        }
+        return;
+    }
+    const unsigned per = (unsigned)(gw * gh);
+    const long long plane = PASS == P_FWD ? (long long)p.OH * p.OW : (long long)p.H * p.W;
+    // four pixels of one image side by side, on a boundary of four
+    if (!phased && (plane & 3) == 0 && ((uintptr_t)out & (4 * sizeof(TOut) - 1)) == 0) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int col = n0 + wn * (TN / 2) + j * 16 + 4 * g4;
+            if (col >= ncol) continue;
+            const unsigned n = (unsigned)col / per;
+            TOut *o = out + (long long)n * p.M * plane + (col - n * per);
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                const int m = mlane + 16 * i;
+                if (m >= (int)p.M) continue;
+                TOut r[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) st_f(r, v, acc[i][j][v]);
+                if constexpr (sizeof(TOut) == 4)
+                    *reinterpret_cast<uint4 *>(o + m * plane) = __builtin_bit_cast(uint4, r);
+                else
+                    *reinterpret_cast<uint2 *>(o + m * plane) = __builtin_bit_cast(uint2, r);
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int col = n0 + wn * (TN / 2) + j * 16 + 4 * g4;
+        if (col >= ncol) continue;
+        const unsigned n = (unsigned)col / per, yx = col - n * per;
+        int y = (int)(yx / (unsigned)gw), x = (int)yx - y * gw;
+        long long img = (long long)n * p.M * plane;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const long long at = img + (phased ? (long long)(p.s1 * y + ry) * p.W + p.s0 * x + rx : (long long)y * gw + x);
+            if (col + v < ncol) {
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+                    if (mlane + 16 * i < (int)p.M) st_f(out, at + (mlane + 16 * i) * plane, acc[i][j][v]);
+            }
+            if (++x == gw) {
+                x = 0;
+                if (++y == gh) {
+                    y = 0;
+                    img += p.M * plane;
+                }
+            }
+        }
     }
 }
 
 // ------------------------------------------------------------- kernel
-template <int MODE, typename TIn, typename TOut, int PASS, bool CL = false>
+template <int MODE, typename TIn, typename TOut, int PASS>
 __global__ __launch_bounds__(NT) void nn_gemm(TOut *__restrict__ out, const TIn *__restrict__ in0,
                                               const TIn *__restrict__ in1, float *__restrict__ partial,
                                               NNParams p) {
@@ -634,36 +882,7 @@ __global__ __launch_bounds__(NT) void nn_gemm(TOut *__restrict__ out, const TIn 
     long long ks1 = ks0 + kps;
     if (ks1 > ksteps) ks1 = ksteps;
 
-    if constexpr (CL) {
-        // in0 = the channel-last activation, in1 = the packed weights. A ring
-        // of CL_DEPTH register sets keeps the loads of the next CL_DEPTH - 1
-        // slices in flight while a slice is stored and multiplied.
-        // Every lane issues the same loads in every slot (slices past the
-        // range reload the last one), so the waits before each store count
-        // exactly the CL_DEPTH - 1 slices still in flight.
-        GatherCL<TIn, PASS> g(in0, in1, p, m0 + lrow, n0 + lrow, ph);
-        constexpr int Q = GatherCL<TIn, PASS>::Q;
-        if (ks0 < ks1) {
-            uint4 ra[CL_DEPTH][Q], rb[CL_DEPTH][Q];
-            const long long last = ks1 - 1;
-#pragma unroll
-            for (int d = 0; d < CL_DEPTH; ++d) g.load(min(ks0 + d, last), kk0, ra[d], rb[d]);
-            for (long long ks = ks0; ks < ks1; ks += CL_DEPTH) {
-#pragma unroll
-                for (int d = 0; d < CL_DEPTH; ++d) {
-                    const bool live = ks + d < ks1;
-                    __syncthreads();
-                    if (live) {
-                        store_raw16<MODE>(tA, lrow, kk0, ra[d]);
-                        store_raw16<MODE>(tB, lrow, kk0, rb[d]);
-                    }
-                    __syncthreads();
-                    g.load(min(ks + d + CL_DEPTH, last), kk0, ra[d], rb[d]);
-                    if (live) mma_slice<MODE>(tA, tB, wm, wn, lane, acc);
-                }
-            }
-        }
-    } else {
+    {
         Gather<TIn, PASS> g(in0, in1, p, m0 + lrow, n0 + lrow, ph);
         float va[16], vb[16];
         if (ks0 < ks1) g.load(ks0, kk0, va, vb);
@@ -745,37 +964,46 @@ __global__ __launch_bounds__(NT) void nn_gemm(TOut *__restrict__ out, const TIn 
 // Second stage of a split forward or data gradient: sums the nsplit partial
 // tiles of each output element in split order (deterministic) and stores it
 // in the output layout. Padding columns of the phased layout are skipped.
+// blockIdx.y: output channel; a lane owns columns, 32-bit throughout (the
+// launcher keeps M * Ncol of a split problem below 2^26).
 template <typename TOut, int PASS>
 __global__ __launch_bounds__(256) void nn_split_reduce(TOut *__restrict__ out, const float *__restrict__ partial,
                                                        NNParams p) {
+    const int row = blockIdx.y, nall = (int)p.Ncol;
     const long long total = p.M * p.Ncol;
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < total;
-         e += (long long)gridDim.x * blockDim.x) {
-        const long long row = e / p.Ncol, col = e - row * p.Ncol;
+    const float *src = partial + (long long)row * nall;
+    for (int col = blockIdx.x * 256 + threadIdx.x; col < nall; col += gridDim.x * 256) {
         long long dst;
         if constexpr (PASS == P_FWD) {
-            const Pix q = decode(col, p.OH, p.OW);
-            const long long ohw = (long long)p.OH * p.OW;
-            dst = ((long long)q.n * p.K + row) * ohw + (long long)q.a * p.OW + q.b;
+            const int ohw = p.OH * p.OW, n = col / ohw;
+            dst = ((long long)n * p.K + row) * ohw + (col - n * ohw);
         } else {
-            const long long hw = (long long)p.H * p.W;
+            const int hw = p.H * p.W;
             if (p.phased) {
-                const long long tn = col / BN;
+                const int tn = col / BN;
                 int ph = 0;
                 while (ph + 1 < p.nph && tn >= p.ph_tile0[ph + 1]) ++ph;
-                const long long lc = col - (long long)p.ph_tile0[ph] * BN;
+                const int lc = col - p.ph_tile0[ph] * BN;
                 const int rx = ph % p.s0, ry = ph / p.s0;
                 const int Mx = phase_len(p.W, p.s0, rx), My = phase_len(p.H, p.s1, ry);
-                if (lc >= (long long)p.N * My * Mx) continue;
-                const Pix q = decode(lc, My, Mx);
-                dst = ((long long)q.n * p.C + row) * hw + (long long)(p.s1 * q.a + ry) * p.W + (p.s0 * q.b + rx);
+                if (lc >= p.N * My * Mx) continue;
+                const int n = lc / (My * Mx), yx = lc - n * (My * Mx), y = yx / Mx, x = yx - y * Mx;
+                dst = ((long long)n * p.C + row) * hw + (long long)(p.s1 * y + ry) * p.W + (p.s0 * x + rx);
             } else {
-                const Pix q = decode(col, p.H, p.W);
-                dst = ((long long)q.n * p.C + row) * hw + (long long)q.a * p.W + q.b;
+                const int n = col / hw;
+                dst = ((long long)n * p.C + row) * hw + (col - n * hw);
             }
         }
         float s = 0.f;
-        for (int sp = 0; sp < p.nsplit; ++sp) s += partial[sp * total + e];
+        int sp = 0;
+        for (; sp + 4 <= p.nsplit; sp += 4) {  // four loads in flight, summed in split order
+            float v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = src[(sp + k) * total + col];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s += v[k];
+        }
+        for (; sp < p.nsplit; ++sp) s += src[sp * total + col];
         st_f(out, dst, s);
     }
 }
@@ -908,7 +1136,9 @@ static GemmLayout gemm_layout(const NNParams &p, int pass, int esz, int nsplit) 
     const long long rows = pass == P_FWD ? p.H : p.OH, cols = pass == P_FWD ? p.W : p.OW;
     const long long wb = (long long)p.RS * p.M * Rcp * esz, ab = (long long)p.N * rows * cols * Rcp * esz;
     // the copies are read through buffer resources (32-bit byte offsets)
-    if (esz > 0 && !(env && env[0] == '0') && wb < (1LL << 31) - 64 && ab < (1LL << 31) - 64) {
+    // and columns and rows counted in 32 bits
+    if (esz > 0 && !(env && env[0] == '0') && wb < (1LL << 31) - 64 && ab < (1LL << 31) - 64 &&
+        p.Ncol < (1LL << 30) && p.M < (1LL << 24) && (p.phased || pass == P_FWD || (p.s0 == 1 && p.s1 == 1))) {
         L.cl = 1;
         L.Rcp = (int)Rcp;
         L.wp_bytes = (int)wb;
@@ -943,8 +1173,37 @@ static int gemm_splits(const NNParams &p) {
     }
     while (want > 1 && want * p.M * p.Ncol * 4 > (256LL << 20)) --want;
     if (want > p.ksteps) want = p.ksteps;
-    if (want < 1) want = 1;
+    if (want < 1 || p.M > 65535) want = 1;  // the summing pass counts channels in gridDim.y
     return (int)want;
+}
+
+template <int MODE, typename TIn, typename TOut, int TM, int TN>
+static void cl_launch_tile(int pass, TOut *out, const TIn *act, const TIn *wp, float *part, NNParams &p,
+                           hipStream_t s) {
+    p.tilesM = (p.M + TM - 1) / TM;
+    p.tilesN = (p.Ncol + TN - 1) / TN;
+    auto fn = pass == P_FWD ? nn_clgemm<MODE, TIn, TOut, P_FWD, TM, TN> : nn_clgemm<MODE, TIn, TOut, P_DGRAD, TM, TN>;
+    fn<<<(unsigned)(p.tilesM * p.tilesN * p.nsplit), NT, 0, s>>>(out, act, wp, part, p);
+}
+
+// Wide tiles where they give at least half of the CUs a workgroup, 64 x 64
+// below that (28x28x128x32 -> 128, BF16, 196 wide tiles: 24 us against 29;
+// 14x14x256x32 -> 256, 98 wide tiles: 35 us against 31), and for FP32 at any
+// size: its 64 x 64 tiles keep three or four workgroups per CU to cover the
+// stages' loads, the wide ones two (56x56x64x32 -> 128: 139 us against 164).
+// 64 rows where 128 would leave half of the last tile empty.
+template <int MODE, typename TIn, typename TOut>
+static void cl_launch(int pass, TOut *out, const TIn *act, const TIn *wp, float *part, NNParams &p, hipStream_t s) {
+    const bool half = (p.M - 1) % 128 < 64;
+    const long long wide = (half ? (p.M + 63) / 64 : (p.M + 127) / 128) * ((p.Ncol + 127) / 128) * p.nsplit;
+    if (MODE == M_F32 || 2 * wide < cu_count_current())
+        cl_launch_tile<MODE, TIn, TOut, 64, 64>(pass, out, act, wp, part, p, s);
+    else if constexpr (MODE != M_F32) {
+        if (half)
+            cl_launch_tile<MODE, TIn, TOut, 64, 128>(pass, out, act, wp, part, p, s);
+        else
+            cl_launch_tile<MODE, TIn, TOut, 128, 128>(pass, out, act, wp, part, p, s);
+    }
 }
 
 template <int MODE, typename TIn, typename TOut>
@@ -975,16 +1234,16 @@ static int run(int pass, void *out, const void *a0, const void *a1, NNParams &p,
                 p.act_bytes = L.act_bytes;
                 TIn *wp = (TIn *)(wsb + L.off_w), *act = (TIn *)(wsb + L.off_act);
                 const long long nw = (long long)p.RS * p.M * p.Rcp;
-                const long long b1 = std::min<long long>((nw + 255) / 256, kMaxGridBlocks / 2);
+                const long long b1 = std::min<long long>((nw + 255) / 256, 4096);
                 const int rows = pass == P_FWD ? p.H : p.OH, cols = pass == P_FWD ? p.W : p.OW;
                 const int Cd = pass == P_FWD ? p.C : p.K;
-                const long long na = (long long)p.N * rows * cols * (p.Rcp / (16 / (int)sizeof(TIn)));
-                const long long b2 = std::min<long long>((na + 255) / 256, kMaxGridBlocks / 2);
+                const int npix = p.N * rows * cols;  // below 2^31 / Rcp
+                const int ncg = (p.Rcp * (int)sizeof(TIn) + 127) / 128;
+                const long long b2 = (long long)((npix + 63) / 64) * ncg;
                 nn_cl_copies<TIn><<<(unsigned)(b1 + b2), 256, 0, s>>>(wp, (const TIn *)a1, p, pass == P_DGRAD,
-                                                                      (int)b1, act, (const TIn *)a0, cols, rows,
-                                                                      Cd);
-                auto fn = pass == P_FWD ? nn_gemm<MODE, TIn, TOut, P_FWD, true> : nn_gemm<MODE, TIn, TOut, P_DGRAD, true>;
-                fn<<<grid, NT, smem, s>>>((TOut *)out, act, wp, part, p);
+                                                                      (int)b1, act, (const TIn *)a0, rows * cols, Cd,
+                                                                      npix, ncg);
+                cl_launch<MODE, TIn, TOut>(pass, (TOut *)out, act, wp, part, p, s);
             }
         }
         if (!p.cl) {
@@ -992,10 +1251,8 @@ static int run(int pass, void *out, const void *a0, const void *a1, NNParams &p,
             fn<<<grid, NT, smem, s>>>((TOut *)out, (const TIn *)a0, (const TIn *)a1, part, p);
         }
         if (p.nsplit > 1) {
-            long long blocks = (p.M * p.Ncol + 255) / 256;
-            if (blocks > kMaxGridBlocks) blocks = kMaxGridBlocks;
             auto red = pass == P_FWD ? nn_split_reduce<TOut, P_FWD> : nn_split_reduce<TOut, P_DGRAD>;
-            red<<<dim3((unsigned)blocks), 256, 0, s>>>((TOut *)out, part, p);
+            red<<<dim3((unsigned)((p.Ncol + 255) / 256), (unsigned)p.M), 256, 0, s>>>((TOut *)out, part, p);
         }
     } else {
         if (p.ksteps == 0) {
