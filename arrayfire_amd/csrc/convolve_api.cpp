@@ -18,6 +18,7 @@
 #include "../../include/af/signal.h"
 #include "../../include/afhip_kernels.h"
 #include "autotune.hpp"
+#include "nn_x3.hpp"
 #include "runtime.hpp"
 
 namespace afhip {
@@ -276,6 +277,27 @@ static void run_gemm_split(int pass, const ArrayImpl &in, const ArrayImpl &w, af
             pass == 0 ? "convolve2_nn" : "convolve2_gradient_nn");
 }
 
+// FP32 on the BF16 matrix cores in three parts per operand: f32 arrays at
+// their own precision. AFHIP_NN_X3=0 leaves it out, =1 takes it wherever it
+// serves.
+static int x3_env() {
+    const char *e = std::getenv("AFHIP_NN_X3");
+    return e && (e[0] == '0' || e[0] == '1') ? e[0] - '0' : -1;
+}
+static bool x3_serves(int pass, const ArrayImpl &in, int precision, const NNGeom &g) {
+    if (in.type != f32 || (precision != AFHIP_PRECISION_DEFAULT && precision != AFHIP_PRECISION_F32)) return false;
+    const char *gather = std::getenv("AFHIP_NN_GATHER");
+    if (x3_env() == 0 || (gather && gather[0] == '1')) return false;
+    return nn_x3_workspace(pass, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, 1) > 0;
+}
+static void run_x3(int pass, const ArrayImpl &in, const ArrayImpl &w, void *out, const NNGeom &g, int nsplit) {
+    const long long need = nn_x3_workspace(pass, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, nsplit);
+    auto ws = scratch((size_t)need);
+    check_k(nn_x3(pass, out, in.data(), w.data(), g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, nsplit, ws->ptr, need,
+                  stream()),
+            pass == 0 ? "convolve2_nn" : "convolve2_gradient_nn");
+}
+
 static void run_patch_kernels(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype out_type, int precision,
                               void *out, const NNGeom &g, long long need) {
     auto ws = scratch((size_t)need);
@@ -294,6 +316,9 @@ static std::vector<std::function<void()>> nn_candidates(int pass, const ArrayImp
     if (first) c.push_back(std::move(first));
     const dim4 &o = pass == 0 ? g.y : g.x;
     const long long tiles = (o[2] + 127) / 128 * ((o[0] * o[1] * o[3] + 127) / 128);
+    if (x3_serves(pass, in, precision, g))
+        for (int sp : {1, 2, 4})
+            if (sp == 1 || tiles < device_cus()) c.push_back([=, &in, &w, &g] { run_x3(pass, in, w, out, g, sp); });
     for (int sp : kSplitCands)
         if (sp == 1 || tiles < device_cus())
             c.push_back([=, &in, &w, &g] { run_gemm_split(pass, in, w, out_type, precision, out, g, sp); });
@@ -313,6 +338,10 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
     const long long need = afhip_k_conv2_nn_patch_workspace(pass, in.type, precision, g.x.d, g.w.d,
                                                             g.y.d, g.st, g.pd, g.dl);
     if (need <= 0) return false;
+    if (x3_env() == 1 && x3_serves(pass, in, precision, g)) {
+        run_x3(pass, in, w, out, g, 1);
+        return true;
+    }
     auto patch = [=, &in, &w, &g] { run_patch_kernels(pass, in, w, out_type, precision, out, g, need); };
     const char *sm = std::getenv("AFHIP_NN_SMALL");
     if (sm && sm[0] == '0') {
@@ -320,7 +349,7 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
         return true;
     }
     const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, patch);
-    int c = nn_pick(nn_key("nn2", pass, in, out_type, precision, g), cands);
+    int c = nn_pick(nn_key("nn3", pass, in, out_type, precision, g), cands);
     if (c < 0) {
         const long long tiles = afhip_k_conv2_nn_patch_tiles(pass, in.type, precision, g.x.d, g.w.d, g.y.d, g.st,
                                                              g.pd, g.dl);
@@ -338,9 +367,13 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
 // the built-in choice when the autotuner is off.
 static void run_gemm(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype out_type, int precision,
                      void *out, const NNGeom &g, std::function<void()> first = nullptr) {
+    if (x3_env() == 1 && x3_serves(pass, in, precision, g)) {
+        run_x3(pass, in, w, out, g, 1);
+        return;
+    }
     const bool has_first = (bool)first;
     const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, std::move(first));
-    int c = nn_pick(nn_key("nn_gemm2", pass, in, out_type, precision, g), cands);
+    int c = nn_pick(nn_key("nn_gemm3", pass, in, out_type, precision, g), cands);
     if (c < 0 && has_first) c = 0;
     if (c >= 0)
         cands[c]();

@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "kcommon.hpp"
+#include "../nn_x3.hpp"
 #include "../../../include/afhip_kernels.h"
 
 namespace afhip {
@@ -551,6 +552,123 @@ __device__ inline TapAxis tap_axis(bool fwd, bool phased, int f, int pd, int d, 
     return a;
 }
 
+// A workgroup's tile: split, first channel and column, its stride phase and
+// pixel grid.
+struct ClTile {
+    int split, m0, n0, ph, rx, ry, gw, gh, ncol;
+    bool phased;
+};
+template <int PASS, int TM, int TN>
+__device__ __forceinline__ ClTile cl_tile(const NNParams &p) {
+    ClTile t;
+    const unsigned tiles = (unsigned)(p.tilesM * p.tilesN), bid = blockIdx.x;
+    t.split = (int)(bid / tiles);
+    const unsigned tl = bid - t.split * tiles;
+    const int tm = (int)(tl / (unsigned)p.tilesN), tn = (int)(tl - tm * (unsigned)p.tilesN);
+    t.m0 = tm * TM;
+    t.n0 = tn * TN;
+    t.phased = PASS == P_DGRAD && p.phased;
+    t.ph = t.rx = t.ry = 0;
+    if (t.phased) {  // phases start on whole tiles of BN columns
+        while (t.ph + 1 < p.nph && t.n0 >= p.ph_tile0[t.ph + 1] * BN) ++t.ph;
+        t.n0 -= p.ph_tile0[t.ph] * BN;
+        t.rx = t.ph % p.s0;
+        t.ry = t.ph / p.s0;
+        t.gw = phase_len(p.W, p.s0, t.rx);
+        t.gh = phase_len(p.H, p.s1, t.ry);
+    } else {
+        t.gw = PASS == P_FWD ? p.OW : p.W;
+        t.gh = PASS == P_FWD ? p.OH : p.H;
+    }
+    t.ncol = p.N * t.gw * t.gh;  // columns of the grid
+    return t;
+}
+
+// Results of a wave's TM/2 x TN/2 block, to the split's partial tile or to the
+// output.
+template <typename TOut, int PASS, int TM, int TN>
+__device__ __forceinline__ void cl_store(TOut *__restrict__ out, float *__restrict__ partial,
+                                         const f32x4_t (&acc)[TM / 32][TN / 32], const NNParams &p, const ClTile &t,
+                                         int wm, int wn, int r16, int g4) {
+    constexpr int MI = TM / 32, NJ = TN / 32;
+    const int m0 = t.m0, n0 = t.n0, ph = t.ph, rx = t.rx, ry = t.ry, gw = t.gw, gh = t.gh, ncol = t.ncol;
+    const bool phased = t.phased;
+    const int split = t.split;
+    // acc[i][j][v]: channel m0 + wm*TM/2 + i*16 + r16, column n0 + wn*TN/2 + j*16 + 4*g4 + v
+    const int mlane = m0 + wm * (TM / 2) + r16;
+    if (p.nsplit > 1) {
+        const int pc0 = phased ? p.ph_tile0[ph] * BN : 0, nall = (int)p.Ncol;
+        float *pt = partial + (long long)split * p.M * p.Ncol;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int col = pc0 + n0 + wn * (TN / 2) + j * 16 + 4 * g4;
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                const int m = mlane + 16 * i;
+                if (m >= (int)p.M) continue;
+                float *o = pt + (long long)m * nall + col;
+                if ((nall & 3) == 0 && col + 4 <= nall) {
+                    *reinterpret_cast<float4 *>(o) = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (col + v < nall) o[v] = acc[i][j][v];
+                }
+            }
+        }
+        return;
+    }
+    const unsigned per = (unsigned)(gw * gh);
+    const long long plane = PASS == P_FWD ? (long long)p.OH * p.OW : (long long)p.H * p.W;
+    // four pixels of one image side by side, on a boundary of four
+    if (!phased && (plane & 3) == 0 && ((uintptr_t)out & (4 * sizeof(TOut) - 1)) == 0) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int col = n0 + wn * (TN / 2) + j * 16 + 4 * g4;
+            if (col >= ncol) continue;
+            const unsigned n = (unsigned)col / per;
+            TOut *o = out + (long long)n * p.M * plane + (col - n * per);
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                const int m = mlane + 16 * i;
+                if (m >= (int)p.M) continue;
+                TOut r[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) st_f(r, v, acc[i][j][v]);
+                if constexpr (sizeof(TOut) == 4)
+                    *reinterpret_cast<uint4 *>(o + m * plane) = __builtin_bit_cast(uint4, r);
+                else
+                    *reinterpret_cast<uint2 *>(o + m * plane) = __builtin_bit_cast(uint2, r);
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int col = n0 + wn * (TN / 2) + j * 16 + 4 * g4;
+        if (col >= ncol) continue;
+        const unsigned n = (unsigned)col / per, yx = col - n * per;
+        int y = (int)(yx / (unsigned)gw), x = (int)yx - y * gw;
+        long long img = (long long)n * p.M * plane;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const long long at = img + (phased ? (long long)(p.s1 * y + ry) * p.W + p.s0 * x + rx : (long long)y * gw + x);
+            if (col + v < ncol) {
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+                    if (mlane + 16 * i < (int)p.M) st_f(out, at + (mlane + 16 * i) * plane, acc[i][j][v]);
+            }
+            if (++x == gw) {
+                x = 0;
+                if (++y == gh) {
+                    y = 0;
+                    img += p.M * plane;
+                }
+            }
+        }
+    }
+}
+
 // Output tile TM x TN per 256-lane workgroup, 2 x 2 waves. R is walked in
 // stages of 128 bytes per row: two 32-deep slices of 16-bit operands, one of
 // FP32, in the slice order of nn_gemm, so both give the same bits. LDS rows
@@ -581,34 +699,16 @@ __global__ __launch_bounds__(NT, 2) void nn_clgemm(TOut *__restrict__ out, const
     constexpr int MI = TM / 32, NJ = TN / 32;               // 16 x 16 results per wave
     __shared__ __attribute__((aligned(16))) char lds[2][(TM + TN) * SB];
 
-    const unsigned tiles = (unsigned)(p.tilesM * p.tilesN);
-    const unsigned bid = blockIdx.x;
-    const int split = (int)(bid / tiles);
-    const unsigned tl = bid - split * tiles;
-    const int tm = (int)(tl / (unsigned)p.tilesN), tn = (int)(tl - tm * (unsigned)p.tilesN);
-    const int m0 = tm * TM;
-    const bool phased = PASS == P_DGRAD && p.phased;
-    int ph = 0, n0 = tn * TN;
-    int rx = 0, ry = 0, gw, gh;  // the tile's pixel grid
-    if (phased) {  // phases start on whole tiles of BN columns
-        while (ph + 1 < p.nph && n0 >= p.ph_tile0[ph + 1] * BN) ++ph;
-        n0 -= p.ph_tile0[ph] * BN;
-        rx = ph % p.s0;
-        ry = ph / p.s0;
-        gw = phase_len(p.W, p.s0, rx);
-        gh = phase_len(p.H, p.s1, ry);
-    } else {
-        gw = PASS == P_FWD ? p.OW : p.W;
-        gh = PASS == P_FWD ? p.OH : p.H;
-    }
+    const ClTile t0 = cl_tile<PASS, TM, TN>(p);
+    const int split = t0.split, m0 = t0.m0, n0 = t0.n0, rx = t0.rx, ry = t0.ry, gw = t0.gw, gh = t0.gh, ncol = t0.ncol;
+    const bool phased = t0.phased;
+    if (n0 >= ncol) return;  // a phase's padding
     const TapAxis ax = tap_axis(PASS == P_FWD, phased, p.fw, p.p0, p.d0, p.s0, rx);
     const TapAxis ay = tap_axis(PASS == P_FWD, phased, p.fh, p.p1, p.d1, p.s1, ry);
     const int slices = ax.n * ay.n * p.kchunks;
     const int kps = phased ? (slices + p.nsplit - 1) / p.nsplit : (int)p.ksteps_per_split;
     const int q0 = split * kps, q1 = min(q0 + kps, slices);
     const int cols = PASS == P_FWD ? p.W : p.OW, rows = PASS == P_FWD ? p.H : p.OH;
-    const int ncol = p.N * gw * gh;  // columns of the grid
-    if (n0 >= ncol) return;          // a phase's padding
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int grp = tid & (G - 1), lrow = tid / G;
@@ -763,80 +863,294 @@ __global__ __launch_bounds__(NT, 2) void nn_clgemm(TOut *__restrict__ out, const
         }
     }
 done:
+    cl_store<TOut, PASS, TM, TN>(out, partial, acc, p, t0, wm, wn, r16, g4);
+}
 
-    // acc[i][j][v]: channel m0 + wm*TM/2 + i*16 + r16, column n0 + wn*TN/2 + j*16 + 4*g4 + v
-    const int mlane = m0 + wm * (TM / 2) + r16;
-    if (p.nsplit > 1) {
-        const int pc0 = phased ? p.ph_tile0[ph] * BN : 0, nall = (int)p.Ncol;
-        float *pt = partial + (long long)split * p.M * p.Ncol;
+// ------------------------------------------------- FP32 in three BF16 parts
+// An FP32 value is the sum of three bfloat16 values, x = x1 + x2 + x3 (each the
+// rounding of what the ones before leave; eight significant bits each make the
+// 24 of FP32). A product x*w is the sum of the six part products down to 2^-16
+// of it, x1w1, x1w2, x2w1, x2w2, x1w3, x3w1; the ones left out are 2^-24 of it
+// and below. The BF16 matrix cores form each part product exactly and add 32
+// of them at a time in FP32, at 16 times the rate of the FP32 ones, so six
+// passes take 3/8 of the time, and the sums see fewer roundings than 4-deep
+// FP32 steps: errors against FP64 are a third
+// of the FP32 kernels' (1.4e-7 against 4.3e-7 relative at 576 products per sum,
+// 4.1e-8 against 9.5e-8 at 27).
+// A part product is as good as the FP32 one only while every part is a normal
+// bfloat16 and nothing overflows: for magnitudes 2^-100 .. 2^63 and for zeros.
+// The copies flag every block of values that holds others (infinities, NaNs,
+// denormals, extremes); a tile that reads a flagged block forms its sums again
+// in FP32 from the arrays themselves.
+constexpr unsigned X3_LO = 27u << 23, X3_HI = 190u << 23;
+
+__device__ __forceinline__ bool x3_odd_value(float v) {
+    const unsigned u = __builtin_bit_cast(unsigned, v) & 0x7fffffffu;
+    return u != 0 && u - X3_LO >= X3_HI - X3_LO;
+}
+__device__ __forceinline__ void x3_parts(float v, uint16_t (&h)[3]) {
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int col = pc0 + n0 + wn * (TN / 2) + j * 16 + 4 * g4;
+    for (int k = 0; k < 3; ++k) {
+        h[k] = f32_to_bf16_bits(v);
+        v -= bf16_bits_to_f32(h[k]);
+    }
+}
+
+// Channel-last copies in parts: [..][slice][part][32 channels], zeros past the
+// reduction channels; the first nbw workgroups the weights [RS][M], the others
+// 64 pixels by one slice each. flags: one word per workgroup.
+__global__ __launch_bounds__(256) void nn_x3_copies(uint16_t *__restrict__ wp, const float *__restrict__ w,
+                                                    NNParams p, int dgrad, int nbw, uint16_t *__restrict__ dst,
+                                                    const float *__restrict__ src, int hw, int Cd, int npix,
+                                                    unsigned *__restrict__ flags) {
+    int odd = 0;
+    if ((int)blockIdx.x < nbw) {
+        const int Rc = dgrad ? p.K : p.C, M = (int)p.M;
+        const unsigned total = (unsigned)(p.RS * M) * (unsigned)p.Rcp;
+        for (unsigned e = blockIdx.x * 256u + threadIdx.x; e < total; e += (unsigned)nbw * 256u) {
+            const unsigned mt = e / (unsigned)p.Rcp;
+            const int r = (int)(e - mt * (unsigned)p.Rcp);
+            const int t = (int)(mt / (unsigned)M), m = (int)mt - t * M;
+            float v = 0.f;
+            if (r < Rc) {
+                const int k = dgrad ? r : m, c = dgrad ? m : r;
+                v = w[((long long)k * p.C + c) * p.RS + (p.RS - 1 - t)];
+            }
+            odd |= x3_odd_value(v);
+            uint16_t h[3];
+            x3_parts(v, h);
+            uint16_t *o = wp + ((long long)mt * p.kchunks + (r >> 5)) * 96 + (r & 31);
 #pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                const int m = mlane + 16 * i;
-                if (m >= (int)p.M) continue;
-                float *o = pt + (long long)m * nall + col;
-                if ((nall & 3) == 0 && col + 4 <= nall) {
-                    *reinterpret_cast<float4 *>(o) = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
-                } else {
+            for (int q = 0; q < 3; ++q) o[32 * q] = h[q];
+        }
+    } else {
+        __shared__ unsigned tile[3][64 * 17];
+        const unsigned b = blockIdx.x - nbw;
+        const int pb = (int)(b / (unsigned)p.kchunks), cs = (int)(b - (unsigned)pb * p.kchunks);
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const int pix = min(pb * 64 + lane, npix - 1), n = pix / hw;
+        const float *s = src + (long long)n * Cd * hw + (pix - n * hw);
+        float v[8];
 #pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        if (col + v < nall) o[v] = acc[i][j][v];
-                }
+        for (int u = 0; u < 8; ++u) v[u] = s[(long long)min(cs * 32 + wave * 8 + u, Cd - 1) * hw];
+        uint16_t h[8][3];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const float x = cs * 32 + wave * 8 + u < Cd ? v[u] : 0.f;
+            odd |= x3_odd_value(x);
+            x3_parts(x, h[u]);
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int u = 0; u < 8; u += 2)
+                tile[q][lane * 17 + wave * 4 + u / 2] = h[u][q] | (unsigned)h[u + 1][q] << 16;
+        __syncthreads();
+        // 64 pixels x 3 parts x 4 groups of 16 bytes
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+            const int e = (int)threadIdx.x + 256 * u, px = e / 12, g = e - px * 12;
+            if (pb * 64 + px < npix) {
+                const unsigned *q = tile[g >> 2] + px * 17 + (g & 3) * 4;
+                *reinterpret_cast<uint4 *>(dst + ((long long)(pb * 64 + px) * p.kchunks + cs) * 96 + g * 8) =
+                    make_uint4(q[0], q[1], q[2], q[3]);
             }
         }
-        return;
     }
-    const unsigned per = (unsigned)(gw * gh);
-    const long long plane = PASS == P_FWD ? (long long)p.OH * p.OW : (long long)p.H * p.W;
-    // four pixels of one image side by side, on a boundary of four
-    if (!phased && (plane & 3) == 0 && ((uintptr_t)out & (4 * sizeof(TOut) - 1)) == 0) {
+    odd = __syncthreads_or(odd);
+    if (threadIdx.x == 0) flags[blockIdx.x] = (unsigned)odd;
+}
+
+// As nn_clgemm, one 32-deep slice (three parts, 64 bytes each per row) per
+// stage, one LDS buffer and 64 x 64 tiles: four workgroups per CU cover each
+// other's loads, stores and barriers (a stage is 24 MFMAs per wave, the matrix
+// cores are busy about 40% of the time). x1w1 has accumulators of its own, so
+// that the five small products, 2^-8 of it and below, are not rounded to its
+// last place each time; the two are added at the end. 56x56x64x32 -> 128, 3x3:
+// 112 us with the copies (19 us of them) against 139 us on the FP32 matrix
+// cores, its data gradient 134 against 153. Wider tiles (64 x 128: 117 us, 128 x
+// 128: 112 and 190 us) lose in occupancy what they save in LDS reads; two LDS
+// buffers with one barrier per stage cost a workgroup per CU (121 us).
+constexpr int X3_T = 64;  // tile
+template <int PASS>
+__global__ __launch_bounds__(NT, 2) void nn_x3gemm(float *__restrict__ out, const uint16_t *__restrict__ act,
+                                                   const uint16_t *__restrict__ wp, const unsigned *__restrict__ flags,
+                                                   int nbw, const float *__restrict__ in, const float *__restrict__ w,
+                                                   float *__restrict__ partial, NNParams p) {
+    constexpr int TM = X3_T, TN = X3_T;
+    constexpr int NA = TM / 64, NB = TN / 64, MI = TM / 32, NJ = TN / 32;
+    constexpr int PLANE = (TM + TN) * 64;
+    constexpr int FP = Lds<M_F32>::PITCH;
+    constexpr int LDSB = 3 * PLANE > (TM + TN) * FP * 4 ? 3 * PLANE : (TM + TN) * FP * 4;
+    __shared__ __attribute__((aligned(16))) char lds[LDSB];
+
+    const ClTile t0 = cl_tile<PASS, TM, TN>(p);
+    const int m0 = t0.m0, n0 = t0.n0, gw = t0.gw, gh = t0.gh, ncol = t0.ncol;
+    if (n0 >= ncol) return;  // a phase's padding
+    const TapAxis ax = tap_axis(PASS == P_FWD, t0.phased, p.fw, p.p0, p.d0, p.s0, t0.rx);
+    const TapAxis ay = tap_axis(PASS == P_FWD, t0.phased, p.fh, p.p1, p.d1, p.s1, t0.ry);
+    const int slices = ax.n * ay.n * p.kchunks;
+    const int kps = t0.phased ? (slices + p.nsplit - 1) / p.nsplit : (int)p.ksteps_per_split;
+    const int q0 = t0.split * kps, q1 = min(q0 + kps, slices);
+    const int cols = PASS == P_FWD ? p.W : p.OW, rows = PASS == P_FWD ? p.H : p.OH;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int grp = tid & 3, lrow = tid >> 2;  // 64 rows per load of the workgroup
+    const int pixb = p.kchunks * 192;
+
+    // the flags of what the tile reads: all weights, and the pixel blocks from
+    // its first row's first tap to its last row's last
+    int odd = 0;
+    {
+        const int per = gw * gh, c1 = min(n0 + TN, ncol) - 1;
+        const int na = n0 / per, nb = c1 / per;
+        const int ya = (n0 - na * per) / gw, yb = (c1 - nb * per) / gw, s1 = PASS == P_FWD ? p.s1 : 1;
+        const int ye = ay.start + (ay.n - 1) * ay.step;
+        const int lo = (na * rows + min(max(ya * s1 + min(ay.start, ye), 0), rows - 1)) * cols;
+        const int hi = (nb * rows + min(max(yb * s1 + max(ay.start, ye), 0), rows - 1)) * cols + cols - 1;
+        for (int f = tid; f < nbw; f += NT) odd |= (int)flags[f];
+        const int f1 = nbw + (hi / 64 + 1) * p.kchunks;
+        for (int f = nbw + lo / 64 * p.kchunks + tid; f < f1; f += NT) odd |= (int)flags[f];
+    }
+
+    int pX[NB], pY[NB];
+    unsigned pBase[NB];
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int col = n0 + wn * (TN / 2) + j * 16 + 4 * g4;
-            if (col >= ncol) continue;
-            const unsigned n = (unsigned)col / per;
-            TOut *o = out + (long long)n * p.M * plane + (col - n * per);
+    for (int r = 0; r < NB; ++r) {
+        const int q = n0 + r * 64 + lrow;
+        const unsigned qc = (unsigned)min(q, ncol - 1);
+        const int n = (int)(qc / (unsigned)(gw * gh));
+        const unsigned yx = qc - (unsigned)n * (gw * gh);
+        const int y = (int)(yx / (unsigned)gw), x = (int)yx - y * gw;
+        pX[r] = PASS == P_FWD ? x * p.s0 : x;
+        pY[r] = q < ncol ? (PASS == P_FWD ? y * p.s1 : y) : -(1 << 30);
+        pBase[r] = ((unsigned)(n * rows + (PASS == P_FWD ? y * p.s1 : y)) * cols + pX[r]) * pixb + grp * 16;
+    }
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(wp), (short)0, p.wp_bytes, 0x00020000);
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(act), (short)0, p.act_bytes, 0x00020000);
+    // the walk over (tap, slice), the same for every lane
+    int q = q0, c, ti, tj;
+    {
+        const int u = q / p.kchunks;
+        c = q - u * p.kchunks;
+        tj = ax.n > 0 ? u / ax.n : 0;
+        ti = u - tj * ax.n;
+    }
+    uint4 sa[NA][3], sb[NB][3];
+    auto load = [&] {
+        unsigned past = q < q1 ? 0u : 0x80000000u;  // opaque: no branch around the loads
+        asm volatile("" : "+s"(past));
+        const int t = (ay.i0 + tj * ay.is) * p.fw + ax.i0 + ti * ax.is;
+        const int sx = ax.start + ti * ax.step, sy = ay.start + tj * ay.step;
+        const unsigned woff = (unsigned)(t * (int)p.M + m0 + lrow) * (unsigned)pixb + c * 192 + grp * 16;
 #pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                const int m = mlane + 16 * i;
-                if (m >= (int)p.M) continue;
-                TOut r[4];
+        for (int r = 0; r < NA; ++r) {
+            const unsigned off = (woff + (unsigned)(64 * r * pixb)) | past | (m0 + lrow + 64 * r < (int)p.M ? 0u : 0x80000000u);
 #pragma unroll
-                for (int v = 0; v < 4; ++v) st_f(r, v, acc[i][j][v]);
-                if constexpr (sizeof(TOut) == 4)
-                    *reinterpret_cast<uint4 *>(o + m * plane) = __builtin_bit_cast(uint4, r);
-                else
-                    *reinterpret_cast<uint2 *>(o + m * plane) = __builtin_bit_cast(uint2, r);
+            for (int h = 0; h < 3; ++h)
+                sa[r][h] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(off + 64 * h), 0, 0));
+        }
+        const unsigned soff = (unsigned)((sy * cols + sx) * pixb + c * 192);
+#pragma unroll
+        for (int r = 0; r < NB; ++r) {
+            const bool in = (unsigned)(pX[r] + sx) < (unsigned)cols && (unsigned)(pY[r] + sy) < (unsigned)rows;
+            unsigned off = pBase[r] + soff;
+            off = (in ? off : 0x80000000u) | past;
+#pragma unroll
+            for (int h = 0; h < 3; ++h)
+                sb[r][h] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(off + 64 * h), 0, 0));
+        }
+        ++q;
+        if (++c == p.kchunks) {
+            c = 0;
+            if (++ti == ax.n) {
+                ti = 0;
+                ++tj;
             }
         }
-        return;
-    }
+    };
+    // 64-byte rows, their groups XORed by the row pair
+    char *slot = lds + lrow * 64 + ((grp ^ (lrow >> 1 & 3)) * 16);
+    const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, g4 = lane >> 4;
+    const int sw = (g4 ^ (r16 >> 1 & 3)) * 16;
+    const char *fa = lds + (wm * (TM / 2) + r16) * 64 + sw, *fb = lds + (TM + wn * (TN / 2) + r16) * 64 + sw;
+    f32x4_t acc[MI][NJ], low[MI][NJ];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int col = n0 + wn * (TN / 2) + j * 16 + 4 * g4;
-        if (col >= ncol) continue;
-        const unsigned n = (unsigned)col / per, yx = col - n * per;
-        int y = (int)(yx / (unsigned)gw), x = (int)yx - y * gw;
-        long long img = (long long)n * p.M * plane;
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const long long at = img + (phased ? (long long)(p.s1 * y + ry) * p.W + p.s0 * x + rx : (long long)y * gw + x);
-            if (col + v < ncol) {
+        for (int j = 0; j < NJ; ++j) acc[i][j] = low[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    load();
+    for (int k = q0; k < q1; ++k) {
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 3; ++h) {
+#pragma unroll
+            for (int r = 0; r < NA; ++r) *reinterpret_cast<uint4 *>(slot + h * PLANE + r * 4096) = sa[r][h];
+#pragma unroll
+            for (int r = 0; r < NB; ++r) *reinterpret_cast<uint4 *>(slot + h * PLANE + TM * 64 + r * 4096) = sb[r][h];
+        }
+        load();
+        __syncthreads();
+        bf16x8_t a[MI][3];
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int h = 0; h < 3; ++h) a[i][h] = *reinterpret_cast<const bf16x8_t *>(fa + h * PLANE + i * 1024);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            bf16x8_t b[3];
+#pragma unroll
+            for (int h = 0; h < 3; ++h) b[h] = *reinterpret_cast<const bf16x8_t *>(fb + h * PLANE + j * 1024);
+            // the smallest products first
+            constexpr int PB[5] = {2, 0, 1, 1, 0}, PA[5] = {0, 2, 1, 0, 1};
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[0], a[i][0], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < 5; ++t)
 #pragma unroll
                 for (int i = 0; i < MI; ++i)
-                    if (mlane + 16 * i < (int)p.M) st_f(out, at + (mlane + 16 * i) * plane, acc[i][j][v]);
-            }
-            if (++x == gw) {
-                x = 0;
-                if (++y == gh) {
-                    y = 0;
-                    img += p.M * plane;
-                }
-            }
+                    low[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[PB[t]], a[i][PA[t]], low[i][j], 0, 0, 0);
         }
     }
+
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] += low[i][j];
+    if (__syncthreads_or(odd)) {
+        // the same sums in FP32, element by element from the arrays
+        float *tA = reinterpret_cast<float *>(lds), *tB = tA + TM * FP;
+        const int row = tid & 127, kk0 = (tid >> 7) * 16;
+        Gather<float, PASS> g(in, w, p, m0 + row, n0 + row, t0.ph);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int k = q0; k < q1; ++k) {
+            float va[16], vb[16];
+            g.load(k, kk0, va, vb);
+            __syncthreads();
+            if (row < TM) store_row16<M_F32>(reinterpret_cast<char *>(tA), row, kk0, va);
+            if (row < TN) store_row16<M_F32>(reinterpret_cast<char *>(tB), row, kk0, vb);
+            __syncthreads();
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    const float4 y = *reinterpret_cast<const float4 *>(tA + (wm * (TM / 2) + i * 16 + r16) * FP + h * 16 + 4 * g4);
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) {
+                        const float4 x = *reinterpret_cast<const float4 *>(tB + (wn * (TN / 2) + j * 16 + r16) * FP + h * 16 + 4 * g4);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, y.x, acc[i][j], 0, 0, 0);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, y.y, acc[i][j], 0, 0, 0);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, y.z, acc[i][j], 0, 0, 0);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, y.w, acc[i][j], 0, 0, 0);
+                    }
+                }
+        }
+    }
+    cl_store<float, PASS, TM, TN>(out, partial, acc, p, t0, wm, wn, r16, g4);
 }
 
 // ------------------------------------------------------------- kernel
@@ -1312,6 +1626,80 @@ static int dispatch(int pass, int in_type, int out_type, int precision, void *ou
     }
 #undef GO
     return K_ERR_TYPE;
+}
+
+// ---- FP32 in three BF16 parts
+struct X3Layout {
+    int wp_bytes = 0, act_bytes = 0, nbw = 0, nba = 0, npix = 0;
+    long long off_act = 0, off_flag = 0, off_part = 0, total = 0;
+};
+static bool x3_layout(const NNParams &p, int pass, X3Layout *L) {
+    auto al = [](long long b) { return (b + 255) & ~255LL; };
+    const long long rows = pass == P_FWD ? p.H : p.OH, cols = pass == P_FWD ? p.W : p.OW;
+    const long long wb = (long long)p.RS * p.M * p.kchunks * 192, npix = (long long)p.N * rows * cols;
+    const long long ab = npix * p.kchunks * 192;
+    if (wb >= (1LL << 31) - 64 || ab >= (1LL << 31) - 64 || p.Ncol >= (1LL << 30) || p.M >= (1LL << 24)) return false;
+    if (pass == P_DGRAD && !p.phased && (p.s0 > 1 || p.s1 > 1)) return false;
+    L->wp_bytes = (int)wb;
+    L->act_bytes = (int)ab;
+    L->npix = (int)npix;
+    L->nbw = (int)std::min<long long>((wb / 6 + 255) / 256, 1024);  // every tile reads all of these flags
+    L->nba = (int)((npix + 63) / 64 * p.kchunks);
+    L->off_act = al(wb);
+    L->off_flag = L->off_act + al(ab);
+    L->off_part = L->off_flag + al(4LL * (L->nbw + L->nba));
+    L->total = L->off_part + (p.nsplit > 1 ? (long long)p.nsplit * p.M * p.Ncol * 4 : 0);
+    return true;
+}
+
+static int x3_setup(NNParams &p, X3Layout *L, int pass, const long long *xd, const long long *wd, const long long *yd,
+                    const long long *st, const long long *pd, const long long *dl, int nsplit) {
+    if (pass != P_FWD && pass != P_DGRAD) return K_ERR_ARG;
+    const int rc = setup(p, pass, xd, wd, yd, st, pd, dl);
+    if (rc) return rc;
+    if (p.M == 0 || p.Ncol == 0 || p.kchunks == 0) return K_ERR_NOT_SUPPORTED;
+    p.nsplit_req = nsplit > 0 ? nsplit : 1;
+    p.nsplit = gemm_splits(p);
+    p.ksteps_per_split = (p.ksteps + p.nsplit - 1) / p.nsplit;
+    p.Rcp = p.kchunks * BK;
+    return x3_layout(p, pass, L) ? K_OK : K_ERR_NOT_SUPPORTED;
+}
+
+long long nn_x3_workspace(int pass, const long long *xd, const long long *wd, const long long *yd,
+                          const long long *st, const long long *pd, const long long *dl, int nsplit) {
+    NNParams p;
+    X3Layout L;
+    return x3_setup(p, &L, pass, xd, wd, yd, st, pd, dl, nsplit) == K_OK ? L.total : 0;
+}
+
+int nn_x3(int pass, void *out, const void *in, const void *w, const long long *xd, const long long *wd,
+          const long long *yd, const long long *st, const long long *pd, const long long *dl, int nsplit, void *ws,
+          long long ws_bytes, hipStream_t s) {
+    NNParams p;
+    X3Layout L;
+    const int rc = x3_setup(p, &L, pass, xd, wd, yd, st, pd, dl, nsplit);
+    if (rc) return rc;
+    if (ws == nullptr || ws_bytes < L.total) return K_ERR_ARG;
+    char *b = (char *)ws;
+    uint16_t *wp = (uint16_t *)b, *act = (uint16_t *)(b + L.off_act);
+    unsigned *flags = (unsigned *)(b + L.off_flag);
+    float *part = p.nsplit > 1 ? (float *)(b + L.off_part) : nullptr;
+    p.wp_bytes = L.wp_bytes;
+    p.act_bytes = L.act_bytes;
+    const int rows = pass == P_FWD ? p.H : p.OH, cols = pass == P_FWD ? p.W : p.OW;
+    nn_x3_copies<<<(unsigned)(L.nbw + L.nba), 256, 0, s>>>(wp, (const float *)w, p, pass == P_DGRAD, L.nbw, act,
+                                                          (const float *)in, rows * cols, pass == P_FWD ? p.C : p.K,
+                                                          L.npix, flags);
+    p.tilesM = (p.M + X3_T - 1) / X3_T;
+    p.tilesN = (p.Ncol + X3_T - 1) / X3_T;
+    auto fn = pass == P_FWD ? nn_x3gemm<P_FWD> : nn_x3gemm<P_DGRAD>;
+    fn<<<(unsigned)(p.tilesM * p.tilesN * p.nsplit), NT, 0, s>>>((float *)out, act, wp, flags, L.nbw, (const float *)in,
+                                                                 (const float *)w, part, p);
+    if (p.nsplit > 1) {
+        auto red = pass == P_FWD ? nn_split_reduce<float, P_FWD> : nn_split_reduce<float, P_DGRAD>;
+        red<<<dim3((unsigned)((p.Ncol + 255) / 256), (unsigned)p.M), 256, 0, s>>>((float *)out, part, p);
+    }
+    return launch_status();
 }
 
 }  // namespace afhip

@@ -1,0 +1,86 @@
+"""FP32 layers on the BF16 matrix cores in three parts per operand
+(AFHIP_NN_X3=1) against FP64: sizes around the 64 x 64 tile and the 32-deep
+slice, strides with phases (some without taps), dilation, splits by the
+autotuner's route left alone. The bar is half of the 1e-6 that FP32 sums of
+these lengths stay below, plus: the error may not exceed that of the FP32
+kernels on the same data. Values outside the range in which three parts are
+exact (infinities, NaNs, denormals, extremes) must come out as from the FP32
+kernels."""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+GEOMS = [
+    ((8, 8, 32, 1), (1, 1, 32, 64), (1, 1), (0, 0), (1, 1)),
+    ((13, 10, 33, 2), (3, 3, 33, 65), (1, 1), (1, 1), (1, 1)),
+    ((20, 17, 3, 2), (5, 5, 3, 7), (1, 1), (2, 2), (1, 1)),
+    ((28, 28, 40, 2), (3, 3, 40, 70), (2, 2), (1, 1), (1, 1)),
+    ((25, 20, 16, 1), (3, 2, 16, 70), (6, 5), (0, 1), (1, 1)),
+    ((27, 9, 100, 2), (3, 3, 100, 128), (1, 1), (2, 2), (2, 2)),
+]
+
+
+def _id(g):
+    return "x{}_w{}_s{}_p{}_d{}".format(*["x".join(map(str, v)) for v in g])
+
+
+def _both(af, X, W, DY, g):
+    st, pd, dl = g[2:]
+    y = af.convolve2NN(X, W, st, pd, dl)
+    dx = af.convolve2GradientNN(DY, X, W, y, st, pd, dl, af.AF_CONV_GRADIENT_DATA)
+    return y.to_numpy(), dx.to_numpy()
+
+
+@pytest.mark.parametrize("g", GEOMS, ids=_id)
+def test_against_fp64(af, rng, g, monkeypatch):
+    x = rng.standard_normal(g[0]).astype(np.float32)
+    w = (rng.standard_normal(g[1]) * 0.1).astype(np.float32)
+    y64 = oracle.conv2_nn_direct_f64(x, w, *g[2:])
+    dy = rng.standard_normal(y64.shape).astype(np.float32)
+    dx64 = oracle.conv2_data_grad_direct_f64(dy, x, w, *g[2:])
+    X, W, DY = af.Array(x), af.Array(w), af.Array(dy)
+    monkeypatch.setenv("AFHIP_NN_X3", "1")
+    y, dx = _both(af, X, W, DY, g)
+    monkeypatch.setenv("AFHIP_NN_GATHER", "1")
+    monkeypatch.setenv("AFHIP_NN_SPLIT", "1")
+    y1, dx1 = _both(af, X, W, DY, g)
+    for got, one, ref in ((y, y1, y64), (dx, dx1, dx64)):
+        e = oracle.rel_l2(got, ref)
+        assert e <= 5e-7
+        assert e <= oracle.rel_l2(one, ref) + 1e-8
+        # pixels that no tap reaches are exact zeros
+        assert np.array_equal(got[ref == 0], ref[ref == 0])
+
+
+@pytest.mark.parametrize("what", ["x", "w", "all_tiny"])
+def test_values_out_of_range(af, rng, what, monkeypatch):
+    g = ((30, 26, 40, 2), (3, 3, 40, 70), (1, 1), (1, 1), (1, 1))
+    x = rng.standard_normal(g[0]).astype(np.float32)
+    w = (rng.standard_normal(g[1]) * 0.1).astype(np.float32)
+    dy = rng.standard_normal((30, 26, 70, 2)).astype(np.float32)
+    odd = [np.inf, -np.inf, np.nan, 3e38, -1e30, 1e-38, 1e-42, 2e-35]
+    if what == "x":
+        for k, v in enumerate(odd):
+            x[3 * k, 25 - 3 * k, 5 * k, k % 2] = v
+            dy[29 - 3 * k, 3 * k, 8 * k, k % 2] = v
+    elif what == "w":
+        w[1, 1, 3, 7], w[0, 2, 39, 69], w[2, 0, 0, 64] = np.inf, 1e-40, np.nan
+    else:
+        x *= np.float32(1e-33)
+        dy *= np.float32(1e-33)
+    X, W, DY = af.Array(x), af.Array(w), af.Array(dy)
+    monkeypatch.setenv("AFHIP_NN_X3", "1")
+    got = _both(af, X, W, DY, g)
+    monkeypatch.setenv("AFHIP_NN_GATHER", "1")
+    monkeypatch.setenv("AFHIP_NN_SPLIT", "1")
+    for a, b in zip(got, _both(af, X, W, DY, g)):
+        np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
+        fin = np.isfinite(b)
+        np.testing.assert_array_equal(a[~fin & ~np.isnan(b)], b[~fin & ~np.isnan(b)])
+        if what != "x":  # every tile reads the odd value
+            np.testing.assert_array_equal(a[fin], b[fin])
+        else:
+            np.testing.assert_allclose(a[fin], b[fin], rtol=2e-5, atol=2e-5)
