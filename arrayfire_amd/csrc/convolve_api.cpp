@@ -18,6 +18,7 @@
 #include "../../include/af/signal.h"
 #include "../../include/afhip_kernels.h"
 #include "autotune.hpp"
+#include "nn_wgemm.hpp"
 #include "nn_x3.hpp"
 #include "runtime.hpp"
 
@@ -441,6 +442,67 @@ static af_array conv2_data_grad(const ArrayImpl &dy, const ArrayImpl &x, const A
     return out.release();
 }
 
+// The row-staged kernels where they serve (filter sides 1 and 3), else the
+// element gather.
+static void wgrad_rows_or_gather(const ArrayImpl &dy, const ArrayImpl &x, const NNGeom &g, int precision,
+                                 af_dtype out_type, void *o, bool gather) {
+    const long long rb = gather ? 0
+                                : afhip_k_conv2_nn_wgrad_rows_workspace(x.type, precision, g.x.d, g.w.d, g.y.d, g.st,
+                                                                        g.pd, g.dl);
+    if (rb > 0) {
+        auto ws = scratch((size_t)rb);
+        check_k(afhip_k_conv2_nn_wgrad_rows(x.type, out_type, precision, o, x.data(), dy.data(), g.x.d, g.w.d, g.y.d,
+                                            g.st, g.pd, g.dl, ws->ptr, rb, stream()),
+                "convolve2_gradient_nn");
+        return;
+    }
+    const long long wsb = afhip_k_conv2_nn_wgrad_workspace(g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl);
+    std::shared_ptr<Buffer> ws;
+    if (wsb > 0) ws = scratch((size_t)wsb);
+    check_k(afhip_k_conv2_nn_wgrad(x.type, out_type, precision, o, x.data(), dy.data(), g.x.d, g.w.d, g.y.d, g.st,
+                                   g.pd, g.dl, ws ? ws->ptr : nullptr, wsb, stream()),
+            "convolve2_gradient_nn");
+}
+
+// The autotuned choice between those and the channel-last GEMM with about one,
+// two or four workgroups per CU (56x56x64x32 -> 128, 3x3, BF16: rows 45 us,
+// GEMM 43; 60x60x16x32 -> 16: 52 and 31; 27x27x96x16 -> 128, 5x5: gather 186, GEMM
+// 37). Built-in rule: the
+// row-staged kernels where they serve, else the GEMM. AFHIP_NN_WG=0 leaves the
+// GEMM out, =1 takes it wherever it serves.
+static void run_wgrad(const ArrayImpl &dy, const ArrayImpl &x, const NNGeom &g, int precision, af_dtype out_type,
+                      void *o) {
+    const char *env = std::getenv("AFHIP_NN_GATHER"), *wg = std::getenv("AFHIP_NN_WG");
+    const bool gather = env && env[0] == '1';
+    const bool own = precision == AFHIP_PRECISION_DEFAULT ||
+                     precision == (x.type == f32   ? AFHIP_PRECISION_F32
+                                   : x.type == f16 ? AFHIP_PRECISION_F16
+                                                   : AFHIP_PRECISION_BF16);
+    auto old = [&] { wgrad_rows_or_gather(dy, x, g, precision, out_type, o, gather); };
+    auto gemm = [&](int target) {
+        const long long need = nn_wgemm_workspace(x.type, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, target);
+        auto ws = scratch((size_t)need);
+        check_k(nn_wgemm(x.type, out_type, o, x.data(), dy.data(), g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, target,
+                         ws->ptr, need, stream()),
+                "convolve2_gradient_nn");
+    };
+    const int cus = device_cus();
+    if (gather || !own || (wg && wg[0] == '0') ||
+        nn_wgemm_workspace(x.type, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, cus) <= 0) {
+        old();
+        return;
+    }
+    if (wg && wg[0] == '1') {
+        gemm(2 * cus);
+        return;
+    }
+    std::vector<std::function<void()>> cands{old, [&] { gemm(cus); }, [&] { gemm(2 * cus); }, [&] { gemm(4 * cus); }};
+    int c = nn_pick(nn_key("nn_wg", 2, x, out_type, precision, g), cands);
+    if (c < 0)
+        c = afhip_k_conv2_nn_wgrad_rows_workspace(x.type, precision, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl) > 0 ? 0 : 2;
+    cands[c]();
+}
+
 // cpu::conv2FilterGradient<T>, src/backend/cpu/convolve.cpp:213-243
 static af_array conv2_filter_grad(const ArrayImpl &dy, const ArrayImpl &x, const ArrayImpl &w,
                                   const NNGeom &g, int precision, af_dtype out_type) {
@@ -457,24 +519,7 @@ static af_array conv2_filter_grad(const ArrayImpl &dy, const ArrayImpl &x, const
                 "convolve2_gradient_nn");
         return out.release();
     }
-    const char *env = std::getenv("AFHIP_NN_GATHER");
-    if (!(env && env[0] == '1')) {
-        const long long rb = afhip_k_conv2_nn_wgrad_rows_workspace(x.type, precision, g.x.d, g.w.d, g.y.d,
-                                                                   g.st, g.pd, g.dl);
-        if (rb > 0) {
-            auto ws = scratch((size_t)rb);
-            check_k(afhip_k_conv2_nn_wgrad_rows(x.type, out_type, precision, o, x.data(), dy.data(), g.x.d,
-                                                g.w.d, g.y.d, g.st, g.pd, g.dl, ws->ptr, rb, stream()),
-                    "convolve2_gradient_nn");
-            return out.release();
-        }
-    }
-    const long long wsb = afhip_k_conv2_nn_wgrad_workspace(g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl);
-    std::shared_ptr<Buffer> ws;
-    if (wsb > 0) ws = scratch((size_t)wsb);
-    check_k(afhip_k_conv2_nn_wgrad(x.type, out_type, precision, o, x.data(), dy.data(), g.x.d, g.w.d,
-                                   g.y.d, g.st, g.pd, g.dl, ws ? ws->ptr : nullptr, wsb, stream()),
-            "convolve2_gradient_nn");
+    run_wgrad(dy, x, g, precision, out_type, o);
     return out.release();
 }
 

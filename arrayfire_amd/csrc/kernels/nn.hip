@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "kcommon.hpp"
+#include "nn_x3_parts.hpp"
 #include "../nn_x3.hpp"
 #include "../../../include/afhip_kernels.h"
 
@@ -882,20 +883,6 @@ done:
 // The copies flag every block of values that holds others (infinities, NaNs,
 // denormals, extremes); a tile that reads a flagged block forms its sums again
 // in FP32 from the arrays themselves.
-constexpr unsigned X3_LO = 27u << 23, X3_HI = 190u << 23;
-
-__device__ __forceinline__ bool x3_odd_value(float v) {
-    const unsigned u = __builtin_bit_cast(unsigned, v) & 0x7fffffffu;
-    return u != 0 && u - X3_LO >= X3_HI - X3_LO;
-}
-__device__ __forceinline__ void x3_parts(float v, uint16_t (&h)[3]) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        h[k] = f32_to_bf16_bits(v);
-        v -= bf16_bits_to_f32(h[k]);
-    }
-}
-
 // Channel-last copies in parts: [..][slice][part][32 channels], zeros past the
 // reduction channels; the first nbw workgroups the weights [RS][M], the others
 // 64 pixels by one slice each. flags: one word per workgroup.
@@ -925,37 +912,7 @@ __global__ __launch_bounds__(256) void nn_x3_copies(uint16_t *__restrict__ wp, c
         }
     } else {
         __shared__ unsigned tile[3][64 * 17];
-        const unsigned b = blockIdx.x - nbw;
-        const int pb = (int)(b / (unsigned)p.kchunks), cs = (int)(b - (unsigned)pb * p.kchunks);
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int pix = min(pb * 64 + lane, npix - 1), n = pix / hw;
-        const float *s = src + (long long)n * Cd * hw + (pix - n * hw);
-        float v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = s[(long long)min(cs * 32 + wave * 8 + u, Cd - 1) * hw];
-        uint16_t h[8][3];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const float x = cs * 32 + wave * 8 + u < Cd ? v[u] : 0.f;
-            odd |= x3_odd_value(x);
-            x3_parts(x, h[u]);
-        }
-#pragma unroll
-        for (int q = 0; q < 3; ++q)
-#pragma unroll
-            for (int u = 0; u < 8; u += 2)
-                tile[q][lane * 17 + wave * 4 + u / 2] = h[u][q] | (unsigned)h[u + 1][q] << 16;
-        __syncthreads();
-        // 64 pixels x 3 parts x 4 groups of 16 bytes
-#pragma unroll
-        for (int u = 0; u < 3; ++u) {
-            const int e = (int)threadIdx.x + 256 * u, px = e / 12, g = e - px * 12;
-            if (pb * 64 + px < npix) {
-                const unsigned *q = tile[g >> 2] + px * 17 + (g & 3) * 4;
-                *reinterpret_cast<uint4 *>(dst + ((long long)(pb * 64 + px) * p.kchunks + cs) * 96 + g * 8) =
-                    make_uint4(q[0], q[1], q[2], q[3]);
-            }
-        }
+        odd = x3_copy_block(dst, src, (int)blockIdx.x - nbw, hw, Cd, npix, p.kchunks, tile);
     }
     odd = __syncthreads_or(odd);
     if (threadIdx.x == 0) flags[blockIdx.x] = (unsigned)odd;
@@ -1638,7 +1595,8 @@ static bool x3_layout(const NNParams &p, int pass, X3Layout *L) {
     const long long rows = pass == P_FWD ? p.H : p.OH, cols = pass == P_FWD ? p.W : p.OW;
     const long long wb = (long long)p.RS * p.M * p.kchunks * 192, npix = (long long)p.N * rows * cols;
     const long long ab = npix * p.kchunks * 192;
-    if (wb >= (1LL << 31) - 64 || ab >= (1LL << 31) - 64 || p.Ncol >= (1LL << 30) || p.M >= (1LL << 24)) return false;
+    // offsets past a resource's end must not wrap
+    if (wb >= (1LL << 30) || ab >= (1LL << 30) || p.Ncol >= (1LL << 30) || p.M >= (1LL << 24)) return false;
     if (pass == P_DGRAD && !p.phased && (p.s0 > 1 || p.s1 > 1)) return false;
     L->wp_bytes = (int)wb;
     L->act_bytes = (int)ab;
