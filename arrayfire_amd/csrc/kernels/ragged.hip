@@ -144,9 +144,11 @@ __global__ __launch_bounds__(RG_THREADS) void ragged_conv2(const RaggedProblem *
             const int ky = e / RG_WP, kx = e % RG_WP;  // padding taps (kx >= FX) are never read
             wf[e] = kx < pr.FX ? pr.filt[(pr.FY - 1 - ky) * pr.FX + (pr.FX - 1 - kx)] : 0.f;
         }
-        load_halo_tile_f32<RG_THREADS, (G::LW + 6) / 4>(tile, pr.in, pr.S0, pr.S1,
-                                                        ox0 + pr.sx - (pr.FX - 1),
-                                                        oy0 + pr.sy - (pr.FY - 1), LH, LW, G::LS);
+        const int ix0 = (int)ox0 + pr.sx - (pr.FX - 1), iy0 = (int)oy0 + pr.sy - (pr.FY - 1);
+        if (halo_rows_ok(pr.S0))
+            load_halo_rows_f32<RG_THREADS, G::LS0 / 4, 8>(tile, pr.in, pr.S0, pr.S1, ix0, iy0, LH, LH, LW, G::LS);
+        else
+            load_halo_tile_f32<RG_THREADS, (G::LW + 6) / 4>(tile, pr.in, pr.S0, pr.S1, ix0, iy0, LH, LW, G::LS);
         __syncthreads();
         float acc[G::TY][G::TX];
 #pragma unroll
@@ -170,9 +172,13 @@ __global__ __launch_bounds__(RG_THREADS) void ragged_conv2(const RaggedProblem *
             const long long oy = oy0 + ty * G::TY + j;
             if (oy >= pr.O1) break;
             float *orow = pr.out + oy * pr.O0;
+            if (oxt + G::TX <= pr.O0) {
+                __builtin_memcpy(orow + oxt, acc[j], 4 * G::TX);  // one store, whatever the alignment
+            } else {
 #pragma unroll
-            for (int i = 0; i < G::TX; ++i)
-                if (oxt + i < pr.O0) orow[oxt + i] = acc[j][i];
+                for (int i = 0; i < G::TX; ++i)
+                    if (oxt + i < pr.O0) orow[oxt + i] = acc[j][i];
+            }
         }
     }
 }

@@ -120,11 +120,15 @@ __global__ __launch_bounds__(256) void sep_fused_f32(float *__restrict__ out,
     const dim_t ox0 = bx * B, oy0 = by * B;
     const dim_t ix0 = ox0 + p.sx - (cf - 1), iy0 = oy0 + p.sy - (rf - 1);
     const int LWr = B + cf - 1, LHr = B + rf - 1;  // halo the filters read
-    load_halo_tile_f32<256, (L + 6) / 4>(xin, in, p.S0, p.S1, ix0, iy0, LHr, LWr, LP);
-    // zero the cells outside the halo (read into registers, never used)
-    for (int i = threadIdx.x; i < L * LP; i += 256) {
-        const int r = i / LP, c = i - (i / LP) * LP;
-        if (r >= LHr || c >= LWr) xin[i] = 0.f;
+    // cells past the halo are read into registers but never used
+    if (halo_rows_ok(p.S0) && p.S1 < (1 << 30)) {
+        load_halo_rows_f32<256, LP / 4, 8>(xin, in, (int)p.S0, (int)p.S1, (int)ix0, (int)iy0, L, LHr, LWr, LP);
+    } else {
+        load_halo_tile_f32<256, (L + 6) / 4>(xin, in, p.S0, p.S1, ix0, iy0, LHr, LWr, LP);
+        for (int i = threadIdx.x; i < L * LP; i += 256) {
+            const int r = i / LP, c = i - (i / LP) * LP;
+            if (r >= LHr || c >= LWr) xin[i] = 0.f;
+        }
     }
     __syncthreads();
 

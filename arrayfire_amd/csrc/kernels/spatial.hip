@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256) void conv2_tile(float *__restrict__ out,
 
     const dim_t ox0 = bx * BX, oy0 = by * BY;
     const dim_t ix0 = ox0 + p.sx - (FX - 1), iy0 = oy0 + p.sy - (FY - 1);
-    load_halo_tile_f32<256, (LW + 6) / 4>(tile, in, p.S0, p.S1, ix0, iy0, LH, LW, LS);
+    load_halo_rows_f32<256, LS / 4, 8>(tile, in, (int)p.S0, (int)p.S1, (int)ix0, (int)iy0, LH, LH, LW, LS);
     __syncthreads();
 
     const int tx = threadIdx.x % NTX, ty = threadIdx.x / NTX;
@@ -193,9 +193,8 @@ __global__ __launch_bounds__(256) void conv2_tile(float *__restrict__ out,
         const dim_t oy = oy0 + ty * TY + j;
         if (oy >= p.O1) break;
         float *orow = out + oy * p.O0;
-        if ((p.O0 & 3) == 0 && oxt + TX <= p.O0) {
-            *reinterpret_cast<float4 *>(orow + oxt) =
-                make_float4(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
+        if (oxt + TX <= p.O0) {  // one 16-byte store, whatever the row's alignment
+            __builtin_memcpy(orow + oxt, acc[j], 16);
         } else {
 #pragma unroll
             for (int i = 0; i < TX; ++i)
@@ -975,7 +974,8 @@ extern "C" int afhip_k_convolve(int dtype, void *out, const long long *odims,
     if (dtype == DT_F32 && rank == 2 && p.batch[1] == 1) {
         const int sx = expand ? 0 : (int)(fdims[0] / 2);
         Tile2Fn strip = strip2_ok(p, in) ? strip2_lookup(fdims[0], fdims[1], sx) : nullptr;
-        Tile2Fn fn = tile2_lookup(fdims[0], fdims[1]);
+        // the tile's loads count in 32 bits
+        Tile2Fn fn = halo_rows_ok(p.sd[0]) && p.sd[1] < (1 << 30) ? tile2_lookup(fdims[0], fdims[1]) : nullptr;
         if (fn || strip) return launch_tile2((float *)out, (const float *)in, (const float *)filt, p, fn, strip, s);
     }
     if (dtype == DT_F32 && rank == 3 && p.batch[1] == 1 && p.batch[2] == 1 && fdims[0] == fdims[1] &&

@@ -149,7 +149,7 @@ AFAPI af_err afhip_ragged_plan_create(afhip_ragged_plan *plan, af_array *outputs
                 q.nbx = q.nby = 0;
                 P.hp.push_back(q);
             }
-            std::string key = "ragged_f32:" + std::to_string(count);
+            std::string key = "ragged2_f32:" + std::to_string(count);
             unsigned long long hsh = 1469598103934665603ull;
             for (const auto &q : P.hp) {
                 const int v[6] = {q.S0, q.S1, q.FX, q.FY, q.sx, q.sy};
