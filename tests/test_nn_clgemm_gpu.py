@@ -54,3 +54,42 @@ def test_same_bits_as_element_gather(af, rng, g, dt, bar, monkeypatch):
     np.testing.assert_array_equal(dx, dx1)
     assert oracle.rel_l2(y, oracle.conv2_nn_direct_f64(x, w, st, pd, dl)) <= bar
     assert oracle.rel_l2(dx, oracle.conv2_data_grad_direct_f64(dy, x, w, st, pd, dl)) <= bar
+
+
+# Results of an unsplit launch leave through LDS. Planes of whole and of broken
+# groups of four pixels, channels one more than and less than a tile's rows,
+# and enough columns for the 64 x 128 and 128 x 128 tiles (FP32 results of the
+# latter leave in two halves).
+STORES = [
+    ((20, 12, 32, 2), (3, 3, 32, 65), (1, 1), (1, 1), (1, 1)),     # 64 x 64, 240-pixel planes
+    ((21, 13, 32, 2), (3, 3, 32, 63), (1, 1), (1, 1), (1, 1)),     # 64 x 64, 273-pixel planes
+    ((64, 67, 16, 4), (3, 3, 16, 63), (1, 1), (1, 1), (1, 1)),     # 64 x 128
+    ((64, 65, 16, 4), (3, 3, 16, 127), (1, 1), (1, 1), (1, 1)),    # 128 x 128
+    ((129, 127, 16, 1), (3, 3, 16, 129), (1, 1), (1, 1), (1, 1)),  # odd planes
+    ((131, 129, 70, 2), (3, 3, 70, 16), (2, 2), (1, 1), (1, 1)),   # data gradient by phases
+]
+
+
+@pytest.mark.parametrize("out", ["f32", "t"])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("g", STORES, ids=lambda g: "x{}_w{}_s{}".format(*["x".join(map(str, v)) for v in g[:3]]))
+def test_unsplit_results(af, rng, g, dt, out, monkeypatch):
+    """The same bits as the element gather, which stores from registers."""
+    t = {"bf16": af.bf16, "f16": af.f16}[dt]
+    ot = af.f32 if out == "f32" else t
+    X = af.Array(rng.standard_normal(g[0]).astype(np.float32)).astype(t)
+    W = af.Array((rng.standard_normal(g[1]) * 0.1).astype(np.float32)).astype(t)
+    monkeypatch.setenv("AFHIP_NN_GATHER", "1")
+    monkeypatch.setenv("AFHIP_NN_SPLIT", "1")
+    y = af.convolve2NN(X, W, *g[2:], out_type=ot)
+    DY = af.Array(np.random.default_rng(7).standard_normal(y.dims).astype(np.float32)).astype(t)
+
+    def both():
+        y = af.convolve2NN(X, W, *g[2:], out_type=ot)
+        dx = af.convolve2GradientNN(DY, X, W, y, *g[2:], af.AF_CONV_GRADIENT_DATA, out_type=ot)
+        return y.astype(af.f32).to_numpy(), dx.astype(af.f32).to_numpy()
+
+    got = both()
+    monkeypatch.setenv("AFHIP_NN_CL", "0")
+    for a, b in zip(got, both()):
+        np.testing.assert_array_equal(a, b)
