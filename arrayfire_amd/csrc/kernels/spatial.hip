@@ -709,12 +709,18 @@ struct Tile3Params {
 
 // FP32 rank-3 kernel for small filters: a 32 x 8 x 8 output block per
 // 256-lane workgroup. The (32+FX-1) x (8+FY-1) x (8+FZ-1) input halo is
-// loaded in one batch of 16-byte loads (every slot's load in flight before
-// any LDS store; rows read as aligned float4s, zeros outside the volume) and
-// scattered into LDS so that tile column c is input column ix0 + c. Each lane
-// computes 4 consecutive x outputs on 2 planes, reading each LDS row segment
-// once (ds_read_b128) for all the taps that touch it; the flipped filter
-// lives in SGPRs.
+// loaded in one batch (every slot's load in flight before any LDS store): one
+// unaligned 16-byte load per four columns where the tile lies inside the rows,
+// four 4-byte ones where it crosses a row's end; addresses are clamped into the
+// volume and what lies outside becomes zero by selects, so no load waits behind
+// a branch. Each lane computes 4 consecutive x outputs on 2 planes, reading
+// each LDS row segment once (ds_read_b128) for all the taps that touch it; the
+// flipped filter lives in SGPRs, for 5x5x5 two slices of it at a time (its 125
+// taps outnumber the SGPRs: kept whole, 115 were spilled to lanes of VGPRs,
+// 248 of which left two waves per SIMD). Bound by the FMAs, small volumes by one
+// round of workgroups. Before, with rows read as aligned float4s behind bounds
+// tests, and now: 192 x 190 x 128, 5x5x5 54.8 and 31.3 us (37 TFLOP/s); 256^3,
+// 5x5x5 179 and 91 us, 3x3x3 50 and 44 us; 128^3, 3x3x3 9.7 and 9.6 us.
 constexpr int T3_BX = 32, T3_BY = 8, T3_BZ = 8;
 
 template <int FX, int FY, int FZ>
@@ -728,11 +734,11 @@ __global__ __launch_bounds__(256) void conv3_tile(float *__restrict__ out,
     constexpr int LS = (((LX + 3) & ~3) * 4) % 64 == 32 ? ((LX + 3) & ~3)
                      : ((((LX + 3) & ~3) + 4) * 4) % 64 == 32 ? ((LX + 3) & ~3) + 4
                      : ((((LX + 3) & ~3) + 8) * 4) % 64 == 32 ? ((LX + 3) & ~3) + 8 : ((LX + 3) & ~3) + 12;
-    constexpr int NQ = (LX + 6) / 4;              // float4 slots per row (origin floored to 4)
+    constexpr int NQ = (LX + 3) / 4;              // groups of four columns per row
     constexpr int SLOTS = LZ * LY * NQ;
     constexpr int NB = (SLOTS + 255) / 256;       // loads per lane, all in flight at once
     constexpr int NV = (4 + FX - 1 + 3) / 4;      // float4 reads per row segment
-    static_assert(4 * 7 + 4 * NV <= LS, "row segment reads stay in the row");
+    static_assert(4 * 7 + 4 * NV <= LS && 4 * NQ <= LS, "row segment reads and stores stay in the row");
     __shared__ __attribute__((aligned(16))) float tile[LZ * LY * LS];
 
     const dim_t blk = xcd_remap(blockIdx.x, p.nblk);
@@ -746,51 +752,47 @@ __global__ __launch_bounds__(256) void conv3_tile(float *__restrict__ out,
     out += b3 * p.out_step3;
     filt += b3 * p.filt_step3;
 
-    float wf[FZ][FY][FX];
-#pragma unroll
-    for (int kz = 0; kz < FZ; ++kz)
-#pragma unroll
-        for (int ky = 0; ky < FY; ++ky)
-#pragma unroll
-            for (int kx = 0; kx < FX; ++kx)
-                wf[kz][ky][kx] = filt[((FZ - 1 - kz) * FY + (FY - 1 - ky)) * FX + (FX - 1 - kx)];
-
     const dim_t ox0 = bx * T3_BX, oy0 = by * T3_BY, oz0 = bz * T3_BZ;
     const dim_t ix0 = ox0 + p.sx - (FX - 1), iy0 = oy0 + p.sy - (FY - 1), iz0 = oz0 + p.sz - (FZ - 1);
-    const dim_t a0 = ix0 - (((ix0 % 4) + 4) % 4);
-    const int off = (int)(ix0 - a0);
-    const bool vec = (p.S0 & 3) == 0;
     {
-        float4 v[NB];
+        f32x4_t v[NB];
+        bool rin[NB];
+        const float *row[NB];
+        int gq[NB];
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
             const int slot = u * 256 + (int)threadIdx.x;
             const int q = slot % NQ, r = (slot / NQ) % LY, z = slot / (NQ * LY);
-            v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-            const dim_t gx = a0 + 4 * q, gy = iy0 + r, gz = iz0 + z;
-            if (slot < SLOTS && gy >= 0 && gy < p.S1 && gz >= 0 && gz < p.S2) {
-                const float *row = in + (gz * p.S1 + gy) * p.S0;
-                if (vec && gx >= 0 && gx + 3 < p.S0) {
-                    v[u] = *reinterpret_cast<const float4 *>(row + gx);
-                } else {
-                    float e4[4];
+            const dim_t gy = iy0 + r, gz = iz0 + z;
+            rin[u] = gy >= 0 && gy < p.S1 && gz >= 0 && gz < p.S2;
+            row[u] = in + (min(max(gz, (dim_t)0), p.S2 - 1) * p.S1 + min(max(gy, (dim_t)0), p.S1 - 1)) * p.S0;
+            gq[u] = 4 * q;
+        }
+        if (ix0 >= 0 && ix0 + 4 * NQ <= p.S0) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) e4[e] = (gx + e >= 0 && gx + e < p.S0) ? row[gx + e] : 0.f;
-                    v[u] = make_float4(e4[0], e4[1], e4[2], e4[3]);
+            for (int u = 0; u < NB; ++u) __builtin_memcpy(&v[u], row[u] + ix0 + gq[u], 16);
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[u][e] = rin[u] ? v[u][e] : 0.f;
+        } else {
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    v[u][e] = row[u][min(max(ix0 + gq[u] + e, (dim_t)0), p.S0 - 1)];
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const dim_t gx = ix0 + gq[u] + e;
+                    v[u][e] = rin[u] && gx >= 0 && gx < p.S0 ? v[u][e] : 0.f;
                 }
-            }
         }
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
             const int slot = u * 256 + (int)threadIdx.x;
-            const int q = slot % NQ, rz = slot / NQ;
-            const int c0 = 4 * q - off;
-            if (slot < SLOTS) {
-                const float e4[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (c0 + e >= 0 && c0 + e < LS) tile[rz * LS + c0 + e] = c0 + e < LX ? e4[e] : 0.f;
-            }
+            if (slot < SLOTS) *reinterpret_cast<f32x4_t *>(tile + (slot / NQ) * LS + gq[u]) = v[u];
         }
     }
     __syncthreads();
@@ -801,31 +803,43 @@ __global__ __launch_bounds__(256) void conv3_tile(float *__restrict__ out,
     for (int k = 0; k < 2; ++k)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[k][i] = 0.f;
+    // w[k]: the slice of the filter that plane k meets in input plane zz
+    float w[2][FY][FX] = {};
+    constexpr int UNROLL = FX * FY * FZ > 64 ? 1 : FZ + 1;
+#pragma unroll UNROLL
+    for (int zz = 0; zz <= FZ; ++zz) {
+        const float *fz = filt + max(FZ - 1 - zz, 0) * (FY * FX);
 #pragma unroll
-    for (int zz = 0; zz < 2 + FZ - 1; ++zz)
+        for (int ky = 0; ky < FY; ++ky)
+#pragma unroll
+            for (int kx = 0; kx < FX; ++kx) {
+                w[1][ky][kx] = w[0][ky][kx];
+                w[0][ky][kx] = fz[(FY - 1 - ky) * FX + (FX - 1 - kx)];
+            }
+        float x[FY][4 * NV];
 #pragma unroll
         for (int ky = 0; ky < FY; ++ky) {
             const float *row = tile + ((2 * tz + zz) * LY + ty + ky) * LS + 4 * tx;
-            float w4[4 * NV];
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
                 const float4 f4 = lds_load16(row + 4 * q);
-                w4[4 * q] = f4.x;
-                w4[4 * q + 1] = f4.y;
-                w4[4 * q + 2] = f4.z;
-                w4[4 * q + 3] = f4.w;
-            }
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                const int kz = zz - k;
-                if (kz >= 0 && kz < FZ) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int kx = 0; kx < FX; ++kx) acc[k][i] = __builtin_fmaf(w4[i + kx], wf[kz][ky][kx], acc[k][i]);
-                }
+                x[ky][4 * q] = f4.x;
+                x[ky][4 * q + 1] = f4.y;
+                x[ky][4 * q + 2] = f4.z;
+                x[ky][4 * q + 3] = f4.w;
             }
         }
+        auto taps = [&](int k) {
+#pragma unroll
+            for (int ky = 0; ky < FY; ++ky)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int kx = 0; kx < FX; ++kx) acc[k][i] = __builtin_fmaf(x[ky][i + kx], w[k][ky][kx], acc[k][i]);
+        };
+        if (zz < FZ) taps(0);
+        if (zz > 0) taps(1);
+    }
 
     const dim_t ox = ox0 + 4 * tx, oy = oy0 + ty;
     if (oy >= p.O1) return;
@@ -979,7 +993,7 @@ extern "C" int afhip_k_convolve(int dtype, void *out, const long long *odims,
         if (fn || strip) return launch_tile2((float *)out, (const float *)in, (const float *)filt, p, fn, strip, s);
     }
     if (dtype == DT_F32 && rank == 3 && p.batch[1] == 1 && p.batch[2] == 1 && fdims[0] == fdims[1] &&
-        fdims[1] == fdims[2] && (fdims[0] == 3 || fdims[0] == 5))
+        fdims[1] == fdims[2] && (fdims[0] == 3 || fdims[0] == 5) && p.sd[0] > 0 && p.sd[1] > 0 && p.sd[2] > 0)
         return launch_tile3((float *)out, (const float *)in, (const float *)filt, p, s);
     // AFHIP_CONV1_TILE=0 in the environment keeps FP32 1-D on conv_generic
     static const bool tile1_off = [] {

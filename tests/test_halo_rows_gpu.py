@@ -1,4 +1,4 @@
-"""The halo loader of the FP32 2-D, fused separable and ragged tile kernels, for
+"""The halo loaders of the FP32 2-D, fused separable, ragged and 3-D tile kernels, for
 rows of any length: narrower than one four-column group, one group more or
 less than a tile of 128 or 64 columns, tiles that cross a row's end, against
 the oracle at 1e-5 relative L2. Infinities next to the border check that
@@ -45,5 +45,22 @@ def test_infinite_columns_stay_in_their_rows(af, rng):
     t = rng.uniform(0.1, 1, (5, 5)).astype(np.float32)
     got = af.convolve2(x, t, 0, SPATIAL).to_numpy()
     ref = oracle.convolve(x, t, 2, False)
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(ref))
+    assert not np.isnan(got).any()
+
+
+@pytest.mark.parametrize("w", [1, 2, 3, 31, 33, 64, 67, 131])
+@pytest.mark.parametrize("h,d", [(1, 2), (7, 9), (17, 8)])
+@pytest.mark.parametrize("f", [3, 5])
+def test_conv3(af, rng, w, h, d, f):
+    x = rng.uniform(-1, 1, (w, h, d)).astype(np.float32)
+    t = rng.uniform(0.1, 1, (f, f, f)).astype(np.float32)
+    for mode in (0, 1):
+        got = af.convolve3(x, t, mode, SPATIAL).to_numpy()
+        assert oracle.rel_l2(got, oracle.convolve(x, t, 3, mode == 1)) <= 1e-5
+    # infinities next to the volume's faces: columns, rows and planes outside
+    # read as zeros, and no tap meets a value that is not its own
+    x[0, 0, d - 1] = x[w - 1, h - 1, 0] = np.inf
+    got, ref = af.convolve3(x, t, 0, SPATIAL).to_numpy(), oracle.convolve(x, t, 3, False)
     np.testing.assert_array_equal(np.isinf(got), np.isinf(ref))
     assert not np.isnan(got).any()
