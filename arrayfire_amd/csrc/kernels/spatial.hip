@@ -121,7 +121,10 @@ struct Tile2Params {
 constexpr int T2_TX = 4, T2_TY = 8, T2_NTX = 32, T2_NTY = 8;
 constexpr int T2_BX = T2_TX * T2_NTX, T2_BY = T2_TY * T2_NTY;
 
-template <int FX, int FY>
+// FAR: images whose rows or columns are past the 32-bit counts of the halo rows
+// loader, by the element loader (a branch between the two in one kernel cost the
+// 9x9 one registers: 262 us against 242 on 60 images of 1023 x 1023).
+template <int FX, int FY, bool FAR>
 __global__ __launch_bounds__(256) void conv2_tile(float *__restrict__ out,
                                                   const float *__restrict__ in,
                                                   const float *__restrict__ filt,
@@ -152,7 +155,10 @@ __global__ __launch_bounds__(256) void conv2_tile(float *__restrict__ out,
 
     const dim_t ox0 = bx * BX, oy0 = by * BY;
     const dim_t ix0 = ox0 + p.sx - (FX - 1), iy0 = oy0 + p.sy - (FY - 1);
-    load_halo_rows_f32<256, LS / 4, 8>(tile, in, (int)p.S0, (int)p.S1, (int)ix0, (int)iy0, LH, LH, LW, LS);
+    if constexpr (FAR)
+        load_halo_tile_f32<256, (LW + 6) / 4>(tile, in, p.S0, p.S1, ix0, iy0, LH, LW, LS);
+    else
+        load_halo_rows_f32<256, LS / 4, 8>(tile, in, (int)p.S0, (int)p.S1, (int)ix0, (int)iy0, LH, LH, LW, LS);
     __syncthreads();
 
     const int tx = threadIdx.x % NTX, ty = threadIdx.x / NTX;
@@ -371,15 +377,15 @@ constexpr int tile2_lds_bytes(int fx, int fy) {
 typedef void (*Tile2Fn)(float *, const float *, const float *, Tile2Params);
 
 template <int FX, int FY>
-constexpr Tile2Fn tile2_entry() {
-    return conv2_tile<FX, FY>;
+constexpr Tile2Fn tile2_entry(bool far) {
+    return far ? conv2_tile<FX, FY, true> : conv2_tile<FX, FY, false>;
 }
 
 // Filter sizes with a register-tiled FP32 2-D variant: every combination up
 // to 5x5, and the odd squares up to 9x9 (larger filters go generic for now).
-static Tile2Fn tile2_lookup(dim_t fx, dim_t fy) {
+static Tile2Fn tile2_lookup(dim_t fx, dim_t fy, bool far) {
 #define T2CASE(a, b) \
-    if (fx == a && fy == b) return tile2_entry<a, b>();
+    if (fx == a && fy == b) return tile2_entry<a, b>(far);
 #define T2ROW(a) T2CASE(a, 1) T2CASE(a, 2) T2CASE(a, 3) T2CASE(a, 4) T2CASE(a, 5)
     T2ROW(1) T2ROW(2) T2ROW(3) T2ROW(4) T2ROW(5)
     T2CASE(7, 7) T2CASE(9, 9)
@@ -988,8 +994,7 @@ extern "C" int afhip_k_convolve(int dtype, void *out, const long long *odims,
     if (dtype == DT_F32 && rank == 2 && p.batch[1] == 1) {
         const int sx = expand ? 0 : (int)(fdims[0] / 2);
         Tile2Fn strip = strip2_ok(p, in) ? strip2_lookup(fdims[0], fdims[1], sx) : nullptr;
-        // the tile's loads count in 32 bits
-        Tile2Fn fn = halo_rows_ok(p.sd[0]) && p.sd[1] < (1 << 30) ? tile2_lookup(fdims[0], fdims[1]) : nullptr;
+        Tile2Fn fn = tile2_lookup(fdims[0], fdims[1], !halo_rows_ok(p.sd[0]) || p.sd[1] >= (1 << 30));
         if (fn || strip) return launch_tile2((float *)out, (const float *)in, (const float *)filt, p, fn, strip, s);
     }
     if (dtype == DT_F32 && rank == 3 && p.batch[1] == 1 && p.batch[2] == 1 && fdims[0] == fdims[1] &&

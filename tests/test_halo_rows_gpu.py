@@ -64,3 +64,14 @@ def test_conv3(af, rng, w, h, d, f):
     got, ref = af.convolve3(x, t, 0, SPATIAL).to_numpy(), oracle.convolve(x, t, 3, False)
     np.testing.assert_array_equal(np.isinf(got), np.isinf(ref))
     assert not np.isnan(got).any()
+
+
+def test_conv2_rows_past_the_loader(af, rng):
+    """Rows of 2^22 columns and more take the older loader, a last tile across
+    the row's end included."""
+    x = rng.random(((1 << 22) + 1, 3), dtype=np.float32)
+    t = rng.uniform(-1, 1, (5, 5)).astype(np.float32)
+    got = af.convolve2(x, t, 0, SPATIAL).to_numpy()
+    assert oracle.rel_l2(got, oracle.convolve(x, t, 2, False)) <= 1e-5
+    cut = slice((1 << 22) - 200, None)
+    assert oracle.rel_l2(got[cut], oracle.convolve(x, t, 2, False)[cut]) <= 1e-5
