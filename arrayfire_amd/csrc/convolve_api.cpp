@@ -392,6 +392,11 @@ static af_array conv2_nn(const ArrayImpl &x, const ArrayImpl &w, const NNGeom &g
                          af_dtype out_type) {
     NewHandle out(make_handle(out_type, g.y));
     if (g.y.elements() == 0) return out.release();
+    // outputs of padding alone: the kernels read at least one pixel and one tap
+    if (g.x.elements() == 0 || g.w.elements() == 0) {
+        check_k(afhip_k_fill(out_type, out.data(), 0.0, g.y.elements(), stream()), "fill");
+        return out.release();
+    }
     if (x.type == f64) {
         check_k(afhip_k_conv2_nn_f64(0, out.data(), x.data(), w.data(), g.x.d, g.w.d, g.y.d, g.st,
                                      g.pd, g.dl, stream()),

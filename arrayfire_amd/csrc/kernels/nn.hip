@@ -1618,6 +1618,8 @@ static bool x3_layout(const NNParams &p, int pass, X3Layout *L) {
     const long long rows = pass == P_FWD ? p.H : p.OH, cols = pass == P_FWD ? p.W : p.OW;
     const long long wb = (long long)p.RS * p.M * p.kchunks * 192, npix = (long long)p.N * rows * cols;
     const long long ab = npix * p.kchunks * 192;
+    // an activation without pixels (outputs of padding alone) has no flags to read
+    if (npix < 1) return false;
     // offsets past a resource's end must not wrap
     if (wb >= (1LL << 30) || ab >= (1LL << 30) || p.Ncol >= (1LL << 30) || p.M >= (1LL << 24)) return false;
     if (pass == P_DGRAD && !p.phased && (p.s0 > 1 || p.s1 > 1)) return false;

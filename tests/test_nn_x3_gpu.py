@@ -84,3 +84,15 @@ def test_values_out_of_range(af, rng, what, monkeypatch):
             np.testing.assert_array_equal(a[fin], b[fin])
         else:
             np.testing.assert_allclose(a[fin], b[fin], rtol=2e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("dims", [(9, 0), (0, 9), (0, 0)], ids=lambda d: "x".join(map(str, d)))
+def test_no_pixels(af, rng, dims, monkeypatch):
+    # padding alone makes outputs: all zeros, whichever kernel is asked for
+    X = af.constant(0, dims + (40, 2))
+    W = af.Array((rng.standard_normal((3, 3, 40, 70)) * 0.1).astype(np.float32))
+    for x3 in ("1", None):
+        monkeypatch.setenv("AFHIP_NN_X3", x3) if x3 else monkeypatch.delenv("AFHIP_NN_X3")
+        y = af.convolve2NN(X, W, (1, 1), (2, 2), (1, 1))
+        assert y.dims == tuple(d + 2 for d in dims) + (70, 2)
+        assert not y.to_numpy().any()
