@@ -64,14 +64,15 @@ __device__ inline float block_max(float v) {
     return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-// Tile and slice of a workgroup; neighbouring tiles on one XCD share halo lines.
+// Tile and slice of a workgroup, `first` being the launch's first tile;
+// neighbouring tiles on one XCD share halo lines.
 struct CannyTile {
     long long slice;
     int i0, j0;
 };
-__device__ inline CannyTile canny_tile(int d0, int d1) {
+__device__ inline CannyTile canny_tile(int d0, int d1, long long first) {
     const int nx = (d0 + CT_W - 1) / CT_W, ny = (d1 + CT_H - 1) / CT_H;
-    const long long b = xcd_remap(blockIdx.x, gridDim.x);
+    const long long b = first + xcd_remap(blockIdx.x, gridDim.x);
     const int per = nx * ny;
     CannyTile t;
     t.slice = b / per;
@@ -83,14 +84,15 @@ __device__ inline CannyTile canny_tile(int d0, int d1) {
 
 template <typename T>
 __global__ __launch_bounds__(256) void canny_suppress_tile(float *__restrict__ sup, float *__restrict__ part,
-                                                           const T *__restrict__ in, int d0, int d1, int is_fast) {
+                                                           const T *__restrict__ in, int d0, int d1, int is_fast,
+                                                           long long first) {
 #pragma clang fp contract(off)
     constexpr int XW = CT_W + 8, XH = CT_H + 8;  // input: +-4
     constexpr int TW = CT_W + 4, TH = CT_H + 8;  // after the dim0 pass: +-2, +-4
     constexpr int SW = CT_W + 4, SH = CT_H + 4;  // smoothed: +-2
     constexpr int MW = CT_W + 2, MH = CT_H + 2;  // magnitude: +-1
     __shared__ float x[XH * XW], tmp[TH * TW], sm[SH * SW], mag[MH * MW];
-    const CannyTile tl = canny_tile(d0, d1);
+    const CannyTile tl = canny_tile(d0, d1, first);
     const int i0 = tl.i0, j0 = tl.j0;
     const T *img = in + tl.slice * ((long long)d0 * d1);
     static_assert(tile_row_holds<XW, XW * XH + 256>() && tile_row_holds<TW, TW * TH>() && tile_row_holds<MW, MW * MH>());
@@ -193,15 +195,16 @@ __global__ __launch_bounds__(256) void canny_suppress_tile(float *__restrict__ s
         top = fmaxf(top, res);
     }
     top = block_max(top);
-    if (threadIdx.x == 0) part[blockIdx.x] = top;
+    if (threadIdx.x == 0) part[first + blockIdx.x] = top;
 }
 
+// A value per workgroup: the largest of its share of part.
 __global__ __launch_bounds__(256) void canny_max_final(float *__restrict__ out, const float *__restrict__ part,
                                                        long long n) {
     float v = 0.f;
-    for (long long e = threadIdx.x; e < n; e += 256) v = fmaxf(v, part[e]);
+    for (long long e = blockIdx.x * 256LL + threadIdx.x; e < n; e += gridDim.x * 256LL) v = fmaxf(v, part[e]);
     v = block_max(v);
-    if (threadIdx.x == 0) out[0] = v;
+    if (threadIdx.x == 0) out[blockIdx.x] = v;
 }
 
 // hist [ns][nbins]: bin = (int)(v / step) clamped to [0, nbins-1]. Counts are
@@ -210,11 +213,12 @@ __global__ __launch_bounds__(256) void canny_max_final(float *__restrict__ out, 
 // would take one at a time.
 constexpr int CH_BINS = 8192;
 __global__ __launch_bounds__(256) void canny_hist_tile(unsigned *__restrict__ hist, const float *__restrict__ v,
-                                                       long long per, int blocks_per_slice, int nbins, float step) {
+                                                       long long per, int blocks_per_slice, int nbins, float step,
+                                                       long long first) {
 #pragma clang fp contract(off)
     extern __shared__ unsigned bins[];
-    const long long sl = blockIdx.x / blocks_per_slice;
-    const int part = (int)(blockIdx.x - sl * blocks_per_slice);
+    const long long b = first + blockIdx.x, sl = b / blocks_per_slice;
+    const int part = (int)(b - sl * blocks_per_slice);
     const bool lds = nbins <= CH_BINS;
     if (lds) {
         for (int b = threadIdx.x; b < nbins; b += 256) bins[b] = 0;
@@ -246,12 +250,12 @@ __global__ __launch_bounds__(256) void canny_hist_tile(unsigned *__restrict__ hi
 // one lane, with its divisions in the chain.
 constexpr int CO_BINS = 4096;
 __global__ __launch_bounds__(256) void canny_otsu_slice(float *__restrict__ thr, const unsigned *__restrict__ hist,
-                                                        int nbins, float total) {
+                                                        int nbins, float total, long long first) {
 #pragma clang fp contract(off)
     __shared__ float w[CO_BINS], m[CO_BINS];
     __shared__ float bk[4];
     __shared__ int bi[4];
-    const unsigned *h = hist + (long long)blockIdx.x * nbins;
+    const unsigned *h = hist + (first + blockIdx.x) * nbins;
     const int t = threadIdx.x;
     for (int b = t; b < nbins; b += 256) {
         const float f = (float)h[b] / total;
@@ -315,7 +319,7 @@ __global__ __launch_bounds__(256) void canny_otsu_slice(float *__restrict__ thr,
     __syncthreads();
     if (t == 0) {
         for (int k = 1; k < 4; ++k) take(bk[k], bi[k]);
-        thr[blockIdx.x] = (float)at;
+        thr[first + blockIdx.x] = (float)at;
     }
 }
 
@@ -371,11 +375,11 @@ __device__ inline void label_join(const S &s, unsigned a, unsigned b) {
 __global__ __launch_bounds__(256) void canny_label_tile(unsigned *__restrict__ labels, const float *__restrict__ sup,
                                                         const float *__restrict__ maxv, int nmax,
                                                         const float *__restrict__ thr, int d0, int d1, float t1,
-                                                        float t2) {
+                                                        float t2, long long first) {
 #pragma clang fp contract(off)
     __shared__ unsigned L[CT_N];
     __shared__ unsigned long long mask[CT_H];
-    const CannyTile tl = canny_tile(d0, d1);
+    const CannyTile tl = canny_tile(d0, d1, first);
     const long long per = (long long)d0 * d1;
     const long long base = tl.slice * per;
     const long long s0 = d0 + 1, s1 = s0 + (long long)(d0 - 1) * (d1 - 1);  // the reference's seed scan
@@ -457,8 +461,9 @@ __global__ __launch_bounds__(256) void canny_label_tile(unsigned *__restrict__ l
 // 2 x 16 its first and last columns: those pixels hold every pair of linear
 // neighbours (the smaller index second) that canny_label_tile has not joined,
 // the pairs that wrap from one column of the image to the next included.
-__global__ __launch_bounds__(128) void canny_label_borders(unsigned *__restrict__ labels, int d0, int d1) {
-    const CannyTile tl = canny_tile(d0, d1);
+__global__ __launch_bounds__(128) void canny_label_borders(unsigned *__restrict__ labels, int d0, int d1,
+                                                           long long first) {
+    const CannyTile tl = canny_tile(d0, d1, first);
     const int t = threadIdx.x;
     int i, j;
     if (t < CT_W) {
@@ -512,18 +517,30 @@ static long long canny_tiles(long long d0, long long d1, long long ns) {
     return (d0 + CT_W - 1) / CT_W * ((d1 + CT_H - 1) / CT_H) * ns;
 }
 
-long long canny_part_floats(long long d0, long long d1, long long ns) { return canny_tiles(d0, d1, ns) + 1; }
+// The tile maxima, then one value or up to 1024.
+constexpr int CT_MAXIMA = 1024;
+long long canny_part_floats(long long d0, long long d1, long long ns) { return canny_tiles(d0, d1, ns) + 1 + CT_MAXIMA; }
+
+// Launches of n workgroups, as many at a time as one launch takes (a batch of
+// very many small images, or an image a few pixels wide, has more tiles).
+template <typename Fn>
+static void canny_launches(long long n, Fn launch) {
+    for (long long first = 0; first < n; first += kMaxGrid256)
+        launch((unsigned)std::min(n - first, kMaxGrid256), first);
+}
 
 template <typename T>
 static void launch_suppress(float *sup, float *part, const void *in, long long d0, long long d1, long long tiles,
                             bool is_fast, hipStream_t s) {
-    canny_suppress_tile<T><<<(unsigned)tiles, 256, 0, s>>>(sup, part, (const T *)in, (int)d0, (int)d1, is_fast);
+    canny_launches(tiles, [&](unsigned nb, long long first) {
+        canny_suppress_tile<T><<<nb, 256, 0, s>>>(sup, part, (const T *)in, (int)d0, (int)d1, is_fast, first);
+    });
 }
 
 int canny_suppress(int dtype, float *sup, CannyMax *top, float *part, const void *in, long long d0, long long d1,
                    long long ns, bool is_fast, bool one, hipStream_t s) {
     const long long tiles = canny_tiles(d0, d1, ns);
-    if (d0 < 2 || d1 < 2 || d0 * d1 >= (1LL << 31) || tiles >= (1LL << 31)) return K_ERR_SIZE;
+    if (d0 < 2 || d1 < 2 || d0 * d1 >= (1LL << 31)) return K_ERR_SIZE;
     switch (dtype) {
         case DT_F32: launch_suppress<float>(sup, part, in, d0, d1, tiles, is_fast, s); break;
         case DT_F64: launch_suppress<double>(sup, part, in, d0, d1, tiles, is_fast, s); break;
@@ -537,13 +554,21 @@ int canny_suppress(int dtype, float *sup, CannyMax *top, float *part, const void
     }
     // the tile kernel of canny_track reduces up to 1024 values itself, which
     // costs each workgroup four loads per lane and saves the launch
-    top->v = part;
-    top->n = (int)tiles;
-    if (one || tiles > 1024) {
-        canny_max_final<<<1, 256, 0, s>>>(part + tiles, part, tiles);
-        top->v = part + tiles;
-        top->n = 1;
+    const float *v = part;
+    long long n = tiles;
+    if (n > 64 * 4 * CT_MAXIMA) {  // too many for one workgroup
+        float *few = part + tiles + 1;
+        canny_max_final<<<CT_MAXIMA, 256, 0, s>>>(few, v, n);
+        v = few;
+        n = CT_MAXIMA;
     }
+    if (one || n > CT_MAXIMA) {
+        canny_max_final<<<1, 256, 0, s>>>(part + tiles, v, n);
+        v = part + tiles;
+        n = 1;
+    }
+    top->v = v;
+    top->n = (int)n;
     return launch_status();
 }
 
@@ -555,26 +580,32 @@ int canny_histogram(unsigned *hist, const float *sup, long long per, long long n
     canny_zero<<<(unsigned)std::min<long long>((nz + 255) / 256, kMaxGridBlocks), 256, 0, s>>>(hist, nz);
     // about 16 values per lane, at most 256 workgroups per slice
     const int bps = (int)std::min<long long>((per + 4095) / 4096, 256);
-    if (ns * bps >= (1LL << 31)) return K_ERR_SIZE;
-    canny_hist_tile<<<(unsigned)(ns * bps), 256, nbins <= CH_BINS ? nbins * sizeof(unsigned) : 0, s>>>(
-        hist, sup, per, bps, nbins, step);
+    canny_launches(ns * bps, [&](unsigned nb, long long first) {
+        canny_hist_tile<<<nb, 256, nbins <= CH_BINS ? nbins * sizeof(unsigned) : 0, s>>>(hist, sup, per, bps, nbins,
+                                                                                        step, first);
+    });
     return launch_status();
 }
 
 // One workgroup per slice up to CO_BINS bins (two LDS arrays), one lane per
 // slice past them.
 int canny_otsu_bins(float *thr, const unsigned *hist, long long per, long long ns, int nbins, hipStream_t s) {
-    if (nbins > CO_BINS || ns >= (1LL << 31)) return canny_otsu_lanes(thr, hist, per, ns, nbins, s);
-    canny_otsu_slice<<<(unsigned)ns, 256, 0, s>>>(thr, hist, nbins, (float)per);
+    if (nbins > CO_BINS) return canny_otsu_lanes(thr, hist, per, ns, nbins, s);
+    canny_launches(ns, [&](unsigned nb, long long first) {
+        canny_otsu_slice<<<nb, 256, 0, s>>>(thr, hist, nbins, (float)per, first);
+    });
     return launch_status();
 }
 
 int canny_track(unsigned char *out, unsigned *labels, const float *sup, CannyMax top, const float *thr,
                 long long d0, long long d1, long long ns, float t1, float t2, hipStream_t s) {
     const long long tiles = canny_tiles(d0, d1, ns), n = d0 * d1 * ns;
-    if (tiles >= (1LL << 31)) return K_ERR_SIZE;
-    canny_label_tile<<<(unsigned)tiles, 256, 0, s>>>(labels, sup, top.v, top.n, thr, (int)d0, (int)d1, t1, t2);
-    canny_label_borders<<<(unsigned)tiles, 128, 0, s>>>(labels, (int)d0, (int)d1);
+    canny_launches(tiles, [&](unsigned nb, long long first) {
+        canny_label_tile<<<nb, 256, 0, s>>>(labels, sup, top.v, top.n, thr, (int)d0, (int)d1, t1, t2, first);
+    });
+    canny_launches(tiles, [&](unsigned nb, long long first) {
+        canny_label_borders<<<nb, 128, 0, s>>>(labels, (int)d0, (int)d1, first);
+    });
     canny_label_out<<<(unsigned)std::min<long long>((n + 255) / 256, kMaxGridBlocks), 256, 0, s>>>(out, labels,
                                                                                                   d0 * d1, n);
     return launch_status();

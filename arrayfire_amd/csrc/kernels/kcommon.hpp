@@ -74,6 +74,9 @@ inline int launch_status() {
 // kernels cap their grid here.
 constexpr int kMaxGridBlocks = 256 * 64;
 
+// The most 256-lane workgroups of one launch: HIP refuses a grid of 2^32 lanes.
+constexpr long long kMaxGrid256 = (1LL << 24) - 1;
+
 // Compute units of the current device (256 on MI355X), cached per device.
 static inline int cu_count_current() {
     static int cus[64] = {0};

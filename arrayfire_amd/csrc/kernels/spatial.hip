@@ -691,7 +691,7 @@ static int launch_whole(void *out, const void *in, const void *filt, const Spati
     t.nbx = (t.O0 + TW_BX - 1) / TW_BX;
     t.nby = (t.O1 + TW_BY - 1) / TW_BY;
     t.nblk = t.nbx * t.nby * p.batch[2] * p.batch[3];
-    if (t.nblk > 0x7fffffffLL) return K_OK;
+    if (t.nblk > kMaxGrid256) return K_OK;  // more tiles than one launch takes
     *served = true;
     if (t.nblk == 0) return K_OK;
     fn<<<dim3((unsigned)t.nblk), dim3(256), 0, s>>>((InT *)out, (const InT *)in, (const float *)filt, t);

@@ -74,3 +74,16 @@ def test_nan_and_inf(af):
     img[20, 10] = np.inf
     img[60, 40] = np.nan
     _check(af, img, 0, 0.1, 0.3)
+
+
+@pytest.mark.parametrize("otsu", [0, 1], ids=["manual", "otsu"])
+def test_more_tiles_than_one_launch_takes(af, otsu):
+    # 2^24 and some images of one tile each; a launch holds fewer workgroups
+    few, times = 997, 16829
+    rng = np.random.default_rng(20261215)
+    base = rng.integers(0, 9, (few, 5, 5), dtype=np.uint8)
+    ref = oracle.canny(np.asfortranarray(base.T), otsu, 0.2, 0.5)
+    assert few * times > 1 << 24 and 0 < ref.mean() < 1
+    img = np.tile(base.reshape(few, 25), (times, 1)).reshape(-1, 5, 5).T
+    got = af.canny(img, otsu, 0.2, 0.5).to_numpy().view(np.uint8).T.reshape(times, -1)
+    assert (got == np.asarray(ref, np.uint8).T.reshape(1, -1)).all()

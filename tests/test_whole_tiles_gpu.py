@@ -59,3 +59,14 @@ def test_sums_past_the_range(af, rng, dt):
     got = _raw(af.convolve2(x, w, 1, SPATIAL).to_numpy())
     ref = _raw(af.convolve2(x, wide, 1, SPATIAL).to_numpy())
     np.testing.assert_array_equal(got, ref[:-1, :-1])
+
+
+def test_more_tiles_than_one_launch_takes(af, rng):
+    # 2^24 and some images of one tile each: the general kernel's grid-stride loop
+    few, times = 997, 16829
+    base, w = rng.integers(0, 100, (few, 2, 2), dtype=np.uint8), _taps(rng, (3, 3), np.uint8)
+    ref = oracle.convolve(np.asfortranarray(base.T), w, 2, False)
+    img = np.tile(base.reshape(few, 4), (times, 1)).reshape(-1, 2, 2).T
+    assert few * times > 1 << 24
+    got = af.convolve2(img, w, 0, SPATIAL).to_numpy().T.reshape(times, -1)
+    assert (got == ref.T.reshape(1, -1)).all()
