@@ -420,8 +420,11 @@ static bool wg_setup(int type, const long long *xd, const long long *wd, const l
     p->dbytes = (int)(npd * p->dpix);
     p->nbx = (int)((npx + 63) / 64 * (x3 ? xs : (xs + 1) / 2));
     p->nbd = (int)((npd + 63) / 64 * (x3 ? ds : (ds + 1) / 2));
-    // three taps share the dy fragments where at most a tenth is wasted
-    *tt = (p->RS + 2) / 3 * 30 <= 11 * p->RS * 3 ? 3 : 1;
+    // three taps share the dy fragments where at most a tenth is wasted, one
+    // tap at a time elsewhere. Three and one, us: 14x14x512x32 -> 512, 1x1, BF16
+    // 32 and 24, FP32 77 and 48; 28x28x128x32 -> 128, 2x2, BF16 28.7 and 26.0,
+    // FP32 55 and 50; 57x57x64x16 -> 64, 4x4, BF16 33.9 and 33.5, FP32 69 and 75.
+    *tt = (p->RS + 2) / 3 * 30 <= 11 * p->RS ? 3 : 1;
     const int SL = x3 ? 1 : 2;
     p->tilesK = (p->K + 63) / 64;
     p->tilesC = (p->C + 63) / 64;

@@ -87,3 +87,15 @@ def test_values_out_of_range(af, rng, what, monkeypatch):
     fin = np.isfinite(b)
     np.testing.assert_array_equal(a[~fin & ~np.isnan(b)], b[~fin & ~np.isnan(b)])
     assert oracle.rel_l2(a[fin], b[fin]) <= 2e-6
+
+
+@pytest.mark.parametrize("taps", [(1, 1), (2, 1), (1, 3), (2, 2), (5, 1), (4, 4)], ids=lambda t: "x".join(map(str, t)))
+@pytest.mark.parametrize("dt,bar", [("f32", 5e-7), ("bf16", 2e-6)], ids=["f32", "bf16"])
+def test_tap_groups(af, rng, taps, dt, bar, monkeypatch):
+    # counts that run tap by tap and in threes, over more than one channel tile
+    t = {"bf16": af.bf16, "f32": af.f32}[dt]
+    g = ((19, 23, 70, 3), taps + (70, 66), (1, 2), (1, 0), (1, 1))
+    X, W, DY = (af.Array(a).astype(t) for a in _data(rng, g))
+    ref = oracle.conv2_filter_grad_direct_f64(*(a.astype(af.f32).to_numpy() for a in (DY, X, W)), *g[2:])
+    monkeypatch.setenv("AFHIP_NN_WG", "1")
+    assert oracle.rel_l2(_dw(af, X, W, DY, g, t), ref) <= bar
