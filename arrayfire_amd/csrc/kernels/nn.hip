@@ -901,44 +901,46 @@ done:
 // FP32 steps: errors against FP64 are a third
 // of the FP32 kernels' (1.4e-7 against 4.3e-7 relative at 576 products per sum,
 // 4.1e-8 against 9.5e-8 at 27).
-// A part product is as good as the FP32 one only while every part is a normal
-// bfloat16 and nothing overflows: for magnitudes 2^-100 .. 2^63 and for zeros.
-// The copies flag every block of values that holds others (infinities, NaNs,
-// denormals, extremes); a tile that reads a flagged block forms its sums again
-// in FP32 from the arrays themselves.
+// The parts hold every value below 2^32 (nn_x3_parts.hpp). The copies flag what
+// their blocks hold; a tile that reads a huge value, an infinity or a NaN, or
+// tiny values and no others (whose results stay the FP32 kernels' to the bit),
+// puts the parts together again and multiplies in FP32 instead.
 // Channel-last copies in parts: [..][slice][part][32 channels], zeros past the
-// reduction channels; the first nbw workgroups the weights [RS][M], the others
-// 64 pixels by one slice each. flags: one word per workgroup.
+// reduction channels; the first nbw workgroups the weights [RS][M], wper of them
+// for each tile's rows, the others 64 pixels by one slice each. flags: one word
+// per workgroup.
+constexpr int X3_T = 64;  // output tile
 __global__ __launch_bounds__(256) void nn_x3_copies(uint16_t *__restrict__ wp, const float *__restrict__ w,
-                                                    NNParams p, int dgrad, int nbw, uint16_t *__restrict__ dst,
-                                                    const float *__restrict__ src, int hw, int Cd, int npix,
-                                                    unsigned *__restrict__ flags) {
-    int odd = 0;
+                                                    NNParams p, int dgrad, int nbw, int wper,
+                                                    uint16_t *__restrict__ dst, const float *__restrict__ src, int hw,
+                                                    int Cd, int npix, unsigned *__restrict__ flags) {
+    int flag = 0;
     if ((int)blockIdx.x < nbw) {
         const int Rc = dgrad ? p.K : p.C, M = (int)p.M;
-        const unsigned total = (unsigned)(p.RS * M) * (unsigned)p.Rcp;
-        for (unsigned e = blockIdx.x * 256u + threadIdx.x; e < total; e += (unsigned)nbw * 256u) {
-            const unsigned mt = e / (unsigned)p.Rcp;
-            const int r = (int)(e - mt * (unsigned)p.Rcp);
-            const int t = (int)(mt / (unsigned)M), m = (int)mt - t * M;
+        const int wt = (int)blockIdx.x / wper, m0 = wt * X3_T, rows = min(X3_T, M - m0);
+        const unsigned total = (unsigned)(p.RS * rows) * (unsigned)p.Rcp;
+        for (unsigned e = (blockIdx.x - wt * wper) * 256u + threadIdx.x; e < total; e += (unsigned)wper * 256u) {
+            const unsigned q = e / (unsigned)p.Rcp;
+            const int r = (int)(e - q * (unsigned)p.Rcp);
+            const int t = (int)(q / (unsigned)rows), m = m0 + (int)q - t * rows;
             float v = 0.f;
             if (r < Rc) {
                 const int k = dgrad ? r : m, c = dgrad ? m : r;
                 v = w[((long long)k * p.C + c) * p.RS + (p.RS - 1 - t)];
             }
-            odd |= x3_odd_value(v);
+            flag |= x3_flag(v);
             uint16_t h[3];
             x3_parts(v, h);
-            uint16_t *o = wp + ((long long)mt * p.kchunks + (r >> 5)) * 96 + (r & 31);
+            uint16_t *o = wp + ((long long)(t * M + m) * p.kchunks + (r >> 5)) * 96 + (r & 31);
 #pragma unroll
-            for (int q = 0; q < 3; ++q) o[32 * q] = h[q];
+            for (int k = 0; k < 3; ++k) o[32 * k] = h[k];
         }
     } else {
         __shared__ unsigned tile[3][64 * 17];
-        odd = x3_copy_block(dst, src, (int)blockIdx.x - nbw, hw, Cd, npix, p.kchunks, tile);
+        flag = x3_copy_block(dst, src, (int)blockIdx.x - nbw, hw, Cd, npix, p.kchunks, tile);
     }
-    odd = __syncthreads_or(odd);
-    if (threadIdx.x == 0) flags[blockIdx.x] = (unsigned)odd;
+    flag = x3_block_flags(flag);
+    if (threadIdx.x == 0) flags[blockIdx.x] = (unsigned)flag;
 }
 
 // As nn_clgemm, one 32-deep slice (three parts, 64 bytes each per row) per
@@ -951,18 +953,14 @@ __global__ __launch_bounds__(256) void nn_x3_copies(uint16_t *__restrict__ wp, c
 // cores, its data gradient 134 against 153. Wider tiles (64 x 128: 117 us, 128 x
 // 128: 112 and 190 us) lose in occupancy what they save in LDS reads; two LDS
 // buffers with one barrier per stage cost a workgroup per CU (121 us).
-constexpr int X3_T = 64;  // tile
 template <int PASS>
 __global__ __launch_bounds__(NT, 2) void nn_x3gemm(float *__restrict__ out, const uint16_t *__restrict__ act,
                                                    const uint16_t *__restrict__ wp, const unsigned *__restrict__ flags,
-                                                   int nbw, const float *__restrict__ in, const float *__restrict__ w,
-                                                   float *__restrict__ partial, NNParams p) {
+                                                   int nbw, int wper, float *__restrict__ partial, NNParams p) {
     constexpr int TM = X3_T, TN = X3_T;
     constexpr int NA = TM / 64, NB = TN / 64, MI = TM / 32, NJ = TN / 32;
     constexpr int PLANE = (TM + TN) * 64;
-    constexpr int FP = Lds<M_F32>::PITCH;
-    constexpr int LDSB = 3 * PLANE > (TM + TN) * FP * 4 ? 3 * PLANE : (TM + TN) * FP * 4;
-    __shared__ __attribute__((aligned(16))) char lds[LDSB];
+    __shared__ __attribute__((aligned(16))) char lds[3 * PLANE];
 
     const ClTile t0 = cl_tile<PASS, TM, TN>(p);
     const int m0 = t0.m0, n0 = t0.n0, gw = t0.gw, gh = t0.gh, ncol = t0.ncol;
@@ -977,9 +975,9 @@ __global__ __launch_bounds__(NT, 2) void nn_x3gemm(float *__restrict__ out, cons
     const int grp = tid & 3, lrow = tid >> 2;  // 64 rows per load of the workgroup
     const int pixb = p.kchunks * 192;
 
-    // the flags of what the tile reads: all weights, and the pixel blocks from
-    // its first row's first tap to its last row's last
-    int odd = 0;
+    // the flags of what the tile reads: its rows' weights, and the pixel blocks
+    // from its first row's first tap to its last row's last
+    int flag = 0;
     {
         const int per = gw * gh, c1 = min(n0 + TN, ncol) - 1;
         const int na = n0 / per, nb = c1 / per;
@@ -987,9 +985,10 @@ __global__ __launch_bounds__(NT, 2) void nn_x3gemm(float *__restrict__ out, cons
         const int ye = ay.start + (ay.n - 1) * ay.step;
         const int lo = (na * rows + min(max(ya * s1 + min(ay.start, ye), 0), rows - 1)) * cols;
         const int hi = (nb * rows + min(max(yb * s1 + max(ay.start, ye), 0), rows - 1)) * cols + cols - 1;
-        for (int f = tid; f < nbw; f += NT) odd |= (int)flags[f];
+        const int wt = m0 / X3_T;
+        for (int f = wt * wper + tid; f < (wt + 1) * wper; f += NT) flag |= (int)flags[f] & X3_HUGE;
         const int f1 = nbw + (hi / 64 + 1) * p.kchunks;
-        for (int f = nbw + lo / 64 * p.kchunks + tid; f < f1; f += NT) odd |= (int)flags[f];
+        for (int f = nbw + lo / 64 * p.kchunks + tid; f < f1; f += NT) flag |= (int)flags[f];
     }
 
     int pX[NB], pY[NB];
@@ -1059,8 +1058,8 @@ __global__ __launch_bounds__(NT, 2) void nn_x3gemm(float *__restrict__ out, cons
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = low[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    load();
-    for (int k = q0; k < q1; ++k) {
+    // parts to LDS, the next stage's loads
+    auto stage = [&] {
         __syncthreads();
 #pragma unroll
         for (int h = 0; h < 3; ++h) {
@@ -1071,6 +1070,12 @@ __global__ __launch_bounds__(NT, 2) void nn_x3gemm(float *__restrict__ out, cons
         }
         load();
         __syncthreads();
+    };
+    load();
+    flag = x3_block_flags(flag);
+    const bool fp32 = (flag & X3_HUGE) || (flag & (X3_TINY | X3_PLAIN)) == X3_TINY;
+    for (int k = fp32 ? q1 : q0; k < q1; ++k) {
+        stage();
         bf16x8_t a[MI][3];
 #pragma unroll
         for (int i = 0; i < MI; ++i)
@@ -1093,41 +1098,42 @@ __global__ __launch_bounds__(NT, 2) void nn_x3gemm(float *__restrict__ out, cons
                     low[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[PB[t]], a[i][PA[t]], low[i][j], 0, 0, 0);
         }
     }
-
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] += low[i][j];
-    if (__syncthreads_or(odd)) {
-        // the same sums in FP32, element by element from the arrays
-        float *tA = reinterpret_cast<float *>(lds), *tB = tA + TM * FP;
-        const int row = tid & 127, kk0 = (tid >> 7) * 16;
-        Gather<float, PASS> g(in, w, p, m0 + row, n0 + row, t0.ph);
+        for (int j = 0; j < NJ; ++j) acc[i][j] = (acc[i][j] + low[i][j]) * X3_UNSCALE;
+    if (fp32) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         for (int k = q0; k < q1; ++k) {
-            float va[16], vb[16];
-            g.load(k, kk0, va, vb);
-            __syncthreads();
-            if (row < TM) store_row16<M_F32>(reinterpret_cast<char *>(tA), row, kk0, va);
-            if (row < TN) store_row16<M_F32>(reinterpret_cast<char *>(tB), row, kk0, vb);
-            __syncthreads();
+            stage();
+            // channels in the order of the FP32 kernels, 4 g4 + e of each half
+            // slice; a pair at a time, for the registers
+#pragma unroll 1
+            for (int h = 0; h < 4; ++h) {
+                const int at = (((h & 2) + (g4 >> 1)) ^ (r16 >> 1 & 3)) * 16 + (g4 & 1) * 8 + (h & 1) * 4 - sw;
+                auto pair = [&](const char *row, float (&v)[2]) {
+                    const unsigned a = *reinterpret_cast<const unsigned *>(row + at),
+                                   b = *reinterpret_cast<const unsigned *>(row + at + PLANE),
+                                   c = *reinterpret_cast<const unsigned *>(row + at + 2 * PLANE);
+                    v[0] = x3_value(a & 0xffff, b & 0xffff, c & 0xffff);
+                    v[1] = x3_value(a >> 16, b >> 16, c >> 16);
+                };
+                float a[MI][2], b[NJ][2];
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+                for (int i = 0; i < MI; ++i) pair(fa + i * 1024, a[i]);
 #pragma unroll
-                for (int i = 0; i < MI; ++i) {
-                    const float4 y = *reinterpret_cast<const float4 *>(tA + (wm * (TM / 2) + i * 16 + r16) * FP + h * 16 + 4 * g4);
+                for (int j = 0; j < NJ; ++j) pair(fb + j * 1024, b[j]);
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j) {
-                        const float4 x = *reinterpret_cast<const float4 *>(tB + (wn * (TN / 2) + j * 16 + r16) * FP + h * 16 + 4 * g4);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, y.x, acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, y.y, acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, y.z, acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, y.w, acc[i][j], 0, 0, 0);
-                    }
-                }
+                for (int e = 0; e < 2; ++e)
+#pragma unroll
+                    for (int i = 0; i < MI; ++i)
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j][e], a[i][e], acc[i][j], 0, 0, 0);
+            }
         }
     }
     cl_store<float, PASS, TM, TN>(out, partial, acc, p, t0, wm, wn, r16, g4, lds);
@@ -1610,7 +1616,7 @@ static int dispatch(int pass, int in_type, int out_type, int precision, void *ou
 
 // ---- FP32 in three BF16 parts
 struct X3Layout {
-    int wp_bytes = 0, act_bytes = 0, nbw = 0, nba = 0, npix = 0;
+    int wp_bytes = 0, act_bytes = 0, wper = 0, nbw = 0, nba = 0, npix = 0;
     long long off_act = 0, off_flag = 0, off_part = 0, total = 0;
 };
 static bool x3_layout(const NNParams &p, int pass, X3Layout *L) {
@@ -1626,7 +1632,10 @@ static bool x3_layout(const NNParams &p, int pass, X3Layout *L) {
     L->wp_bytes = (int)wb;
     L->act_bytes = (int)ab;
     L->npix = (int)npix;
-    L->nbw = (int)std::min<long long>((wb / 6 + 255) / 256, 1024);  // every tile reads all of these flags
+    // weight blocks: a lane per element of a tile's rows, about a thousand in all
+    const long long wt = (p.M + X3_T - 1) / X3_T, each = (long long)p.RS * X3_T * p.kchunks * BK;
+    L->wper = (int)std::max<long long>(1, std::min<long long>((each + 255) / 256, 1024 / wt));
+    L->nbw = (int)wt * L->wper;
     L->nba = (int)((npix + 63) / 64 * p.kchunks);
     L->off_act = al(wb);
     L->off_flag = L->off_act + al(ab);
@@ -1670,14 +1679,14 @@ int nn_x3(int pass, void *out, const void *in, const void *w, const long long *x
     p.wp_bytes = L.wp_bytes;
     p.act_bytes = L.act_bytes;
     const int rows = pass == P_FWD ? p.H : p.OH, cols = pass == P_FWD ? p.W : p.OW;
-    nn_x3_copies<<<(unsigned)(L.nbw + L.nba), 256, 0, s>>>(wp, (const float *)w, p, pass == P_DGRAD, L.nbw, act,
-                                                          (const float *)in, rows * cols, pass == P_FWD ? p.C : p.K,
-                                                          L.npix, flags);
+    nn_x3_copies<<<(unsigned)(L.nbw + L.nba), 256, 0, s>>>(wp, (const float *)w, p, pass == P_DGRAD, L.nbw, L.wper,
+                                                          act, (const float *)in, rows * cols,
+                                                          pass == P_FWD ? p.C : p.K, L.npix, flags);
     p.tilesM = (p.M + X3_T - 1) / X3_T;
     p.tilesN = (p.Ncol + X3_T - 1) / X3_T;
     auto fn = pass == P_FWD ? nn_x3gemm<P_FWD> : nn_x3gemm<P_DGRAD>;
-    fn<<<(unsigned)(p.tilesM * p.tilesN * p.nsplit), NT, 0, s>>>((float *)out, act, wp, flags, L.nbw, (const float *)in,
-                                                                 (const float *)w, part, p);
+    fn<<<(unsigned)(p.tilesM * p.tilesN * p.nsplit), NT, 0, s>>>((float *)out, act, wp, flags, L.nbw, L.wper,
+                                                                 part, p);
     if (p.nsplit > 1) {
         auto red = pass == P_FWD ? nn_split_reduce<float, P_FWD> : nn_split_reduce<float, P_DGRAD>;
         red<<<dim3((unsigned)((p.Ncol + 255) / 256), (unsigned)p.M), 256, 0, s>>>((float *)out, part, p);

@@ -16,7 +16,7 @@
 //
 // f32 arrays run in three BF16 parts per operand (nn_x3_parts.hpp): six part
 // products, the small ones in accumulators of their own; a workgroup that reads
-// a flagged block forms its sums again in FP32 from the arrays.
+// a block with huge values puts the parts together again and multiplies in FP32.
 //
 // us for the call, copies and sum included, against the kernels it replaces or
 // competes with (dims W H C N -> K): BF16 28x28x128x16 -> 128 3x3 stride 2: 20
@@ -64,10 +64,10 @@ __global__ __launch_bounds__(256) void wg_copies(T *__restrict__ xc, T *__restri
     const int slices = first ? p.xs : p.ds;
     if constexpr (sizeof(T) == 4) {
         __shared__ unsigned tile[3][64 * 17];
-        int odd = x3_copy_block(reinterpret_cast<uint16_t *>(first ? xc : dc), first ? x : dy, b, hw, Cd, npix, slices,
-                                tile);
-        odd = __syncthreads_or(odd);
-        if (threadIdx.x == 0) flags[blockIdx.x] = (unsigned)odd;
+        int flag = x3_copy_block(reinterpret_cast<uint16_t *>(first ? xc : dc), first ? x : dy, b, hw, Cd, npix,
+                                 slices, tile);
+        flag = x3_block_flags(flag);
+        if (threadIdx.x == 0) flags[blockIdx.x] = (unsigned)flag;
     } else {
         // 64 pixels x 64 channels through LDS rows of 33 words
         __shared__ unsigned tile[64 * 33];
@@ -97,8 +97,7 @@ __global__ __launch_bounds__(256) void wg_copies(T *__restrict__ xc, T *__restri
 // SL 32-pixel slices per stage, TT taps per workgroup.
 template <int MODE, int SL, int TT>
 __global__ __launch_bounds__(256, 2) void nn_wgemm_k(float *__restrict__ partial, const char *__restrict__ xc,
-                                                     const char *__restrict__ dc, const float *__restrict__ x,
-                                                     const float *__restrict__ dy, const unsigned *__restrict__ flags,
+                                                     const char *__restrict__ dc, const unsigned *__restrict__ flags,
                                                      WgParams p) {
     constexpr int NP = MODE == WG_X3 ? 3 : 1;   // parts
     constexpr int PL = 4096 * SL;               // one part of one operand: 32 SL rows of 128 bytes
@@ -119,7 +118,7 @@ __global__ __launch_bounds__(256, 2) void nn_wgemm_k(float *__restrict__ partial
     const int grp = tid & 7, lrow = tid >> 3;
     const int ohw = p.OH * p.OW;
 
-    int odd = 0;
+    int flag = 0;
     if constexpr (MODE == WG_X3) {
         // the flags of the blocks read: the split's pixels of dy, and of x the
         // rows from its first tap row to its last
@@ -128,8 +127,8 @@ __global__ __launch_bounds__(256, 2) void nn_wgemm_k(float *__restrict__ partial
         const int lo = (na * p.H + min(max(ya * p.s1 - p.p1, 0), p.H - 1)) * p.W;
         const int hi = (nb * p.H + min(max(yb * p.s1 - p.p1 + (p.fh - 1) * p.d1, 0), p.H - 1)) * p.W + p.W - 1;
         const int fx1 = (hi / 64 + 1) * p.xs, fd1 = (b / 64 + 1) * p.ds;
-        for (int f = lo / 64 * p.xs + tid; f < fx1; f += 256) odd |= (int)flags[f];
-        for (int f = a / 64 * p.ds + tid; f < fd1; f += 256) odd |= (int)flags[p.nbx + f];
+        for (int f = lo / 64 * p.xs + tid; f < fx1; f += 256) flag |= (int)flags[f];
+        for (int f = a / 64 * p.ds + tid; f < fd1; f += 256) flag |= (int)flags[p.nbx + f];
     }
 
     // the lane's 16 bytes of a pixel row
@@ -225,22 +224,29 @@ __global__ __launch_bounds__(256, 2) void nn_wgemm_k(float *__restrict__ partial
                 if constexpr (MODE == WG_X3) low[t][i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
             }
 
+    // a stage: pixels to LDS, the next stage's loads, mul per slice
+    auto walk = [&](auto mul) {
+        for (int k = sl0; k < sl1; k += SL) {
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < SL; ++s)
+#pragma unroll
+                for (int h = 0; h < NP; ++h) {
+                    *reinterpret_cast<uint4 *>(slot + h * PL + s * 4096) = sa[s][h];
+#pragma unroll
+                    for (int t = 0; t < TT; ++t)
+                        *reinterpret_cast<uint4 *>(slot + (NP + t * NP + h) * PL + s * 4096) = sb[s][t][h];
+                }
+            load();
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < SL; ++s) mul(s);
+        }
+    };
     load();
-    for (int k = sl0; k < sl1; k += SL) {
-        __syncthreads();
-#pragma unroll
-        for (int s = 0; s < SL; ++s)
-#pragma unroll
-            for (int h = 0; h < NP; ++h) {
-                *reinterpret_cast<uint4 *>(slot + h * PL + s * 4096) = sa[s][h];
-#pragma unroll
-                for (int t = 0; t < TT; ++t)
-                    *reinterpret_cast<uint4 *>(slot + (NP + t * NP + h) * PL + s * 4096) = sb[s][t][h];
-            }
-        load();
-        __syncthreads();
-#pragma unroll
-        for (int s = 0; s < SL; ++s) {
+    if constexpr (MODE == WG_X3) flag = x3_block_flags(flag);
+    if (MODE != WG_X3 || !(flag & X3_HUGE)) {
+        walk([&](int s) {
             s16x8_t a[2][NP];
 #pragma unroll
             for (int i = 0; i < 2; ++i)
@@ -267,65 +273,39 @@ __global__ __launch_bounds__(256, 2) void nn_wgemm_k(float *__restrict__ partial
                             for (int j = 0; j < 2; ++j) low[t][i][j] = mma(a[i][PA[e]], b[j][PB[e]], low[t][i][j]);
                 }
             }
-        }
-    }
-    if constexpr (MODE == WG_X3) {
+        });
+        if constexpr (MODE == WG_X3) {
 #pragma unroll
-        for (int t = 0; t < TT; ++t)
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[t][i][j] += low[t][i][j];
-        if (__syncthreads_or(odd)) {
-            // in FP32 from the arrays, tap by tap: a lane stages eight pixels of
-            // one filter and of one channel
-            constexpr int FP = 36;
-            static_assert(2 * 64 * FP * 4 <= sizeof(lds), "FP32 rows fit the staging buffer");
-            float *tA = reinterpret_cast<float *>(lds), *tB = tA + 64 * FP;
-            const int row = tid >> 2, e0 = (tid & 3) * 8;
-            const long long hw = (long long)p.H * p.W;
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
+            for (int t = 0; t < TT; ++t)
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) acc[t][i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-                for (int k = sl0; k < sl1; ++k) {
-                    float va[8], vb[8];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int qq = k * 32 + e0 + e, qc = min(qq, p.npd - 1);
-                        const int nn = qc / ohw, r = qc - nn * ohw, y = r / p.OW, xx = r - y * p.OW;
-                        const int iy = y * p.s1 - p.p1 + tj[t] * p.d1, ix = xx * p.s0 - p.p0 + ti[t] * p.d0;
-                        va[e] = vb[e] = 0.f;
-                        if (qq < q1 && k0 + row < p.K) va[e] = dy[((long long)nn * p.K + k0 + row) * ohw + r];
-                        if (qq < q1 && c0 + row < p.C && iy >= 0 && iy < p.H && ix >= 0 && ix < p.W)
-                            vb[e] = x[((long long)nn * p.C + c0 + row) * hw + (long long)iy * p.W + ix];
-                    }
-                    __syncthreads();
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        tA[row * FP + e0 + e] = va[e];
-                        tB[row * FP + e0 + e] = vb[e];
-                    }
-                    __syncthreads();
-#pragma unroll
-                    for (int h = 0; h < 8; ++h) {
-                        float a[2], b[2];
-#pragma unroll
-                        for (int i = 0; i < 2; ++i) {
-                            a[i] = tA[(wk * 32 + i * 16 + r16) * FP + 4 * h + g4];
-                            b[i] = tB[(wc * 32 + i * 16 + r16) * FP + 4 * h + g4];
-                        }
-#pragma unroll
-                        for (int i = 0; i < 2; ++i)
-#pragma unroll
-                            for (int j = 0; j < 2; ++j)
-                                acc[t][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[t][i][j], 0, 0, 0);
-                    }
-                }
-            }
+                    for (int j = 0; j < 2; ++j) acc[t][i][j] = (acc[t][i][j] + low[t][i][j]) * X3_UNSCALE;
         }
+    } else if constexpr (MODE == WG_X3) {
+        walk([&](int s) {
+            auto eight = [&](int plane, int blk, float (&v)[8]) {
+                const s16x8_t a = frag(plane + s * 4096, blk), b = frag(plane + PL + s * 4096, blk),
+                              c = frag(plane + 2 * PL + s * 4096, blk);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = x3_value((uint16_t)a[e], (uint16_t)b[e], (uint16_t)c[e]);
+            };
+            float a[2][8];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) eight(0, wk * 2 + i, a[i]);
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    float b[8];
+                    eight((NP + t * NP) * PL, wc * 2 + j, b);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            acc[t][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b[e], acc[t][i][j], 0, 0, 0);
+                }
+        });
     }
 
     // acc[t][i][j][v]: filter k0 + wk*32 + i*16 + 4*g4 + v, channel c0 + wc*32 + j*16 + r16
@@ -478,7 +458,7 @@ int nn_wgemm(int type, int out_type, void *dw, const void *x, const void *dy, co
     auto fn = type == DT_F32    ? (tt == 3 ? nn_wgemm_k<WG_X3, 1, 3> : nn_wgemm_k<WG_X3, 1, 1>)
               : type == DT_BF16 ? (tt == 3 ? nn_wgemm_k<WG_BF16, 2, 3> : nn_wgemm_k<WG_BF16, 2, 1>)
                                 : (tt == 3 ? nn_wgemm_k<WG_F16, 2, 3> : nn_wgemm_k<WG_F16, 2, 1>);
-    fn<<<grid, 256, 0, s>>>(part, xc, dc, (const float *)x, (const float *)dy, flags, p);
+    fn<<<grid, 256, 0, s>>>(part, xc, dc, flags, p);
     const unsigned sb = (unsigned)(((long long)p.RS * p.K * p.C + 63) / 64);
     if (out_type == DT_F32)
         nn_wgemm_sum<float><<<sb, 256, 0, s>>>((float *)dw, part, p);

@@ -1,11 +1,10 @@
 """FP32 layers on the BF16 matrix cores in three parts per operand
 (AFHIP_NN_X3=1) against FP64: sizes around the 64 x 64 tile and the 32-deep
-slice, strides with phases (some without taps), dilation, splits by the
-autotuner's route left alone. The bar is half of the 1e-6 that FP32 sums of
-these lengths stay below, plus: the error may not exceed that of the FP32
-kernels on the same data. Values outside the range in which three parts are
-exact (infinities, NaNs, denormals, extremes) must come out as from the FP32
-kernels."""
+slice, strides with phases (some without taps), dilation. The bar is half of
+the 1e-6 that FP32 sums of these lengths stay below, plus: the error may not
+exceed that of the FP32 kernels on the same data. Values that three parts do
+not hold (infinities, NaNs, magnitudes from 2^32) must come out as from the
+FP32 kernels, and tiles of nothing but tiny values to the bit."""
 import numpy as np
 import pytest
 
@@ -84,6 +83,44 @@ def test_values_out_of_range(af, rng, what, monkeypatch):
             np.testing.assert_array_equal(a[fin], b[fin])
         else:
             np.testing.assert_allclose(a[fin], b[fin], rtol=2e-5, atol=2e-5)
+
+
+def test_tiny_values_among_others(af, rng, monkeypatch):
+    # values far below the others (a saturated softmax's gradient) leave the
+    # tile on the three parts: they add nothing to its sums but the side to
+    # which a tie is rounded, so next to no bit differs from zeros in their
+    # place (from the FP32 kernels' sums half of the values do)
+    g = ((30, 26, 40, 2), (3, 3, 40, 70), (1, 1), (1, 1), (1, 1))
+    x = rng.standard_normal(g[0]).astype(np.float32)
+    w = (rng.standard_normal(g[1]) * 0.1).astype(np.float32)
+    dy = rng.standard_normal((30, 26, 70, 2)).astype(np.float32)
+    at = [rng.random(a.shape) < 0.3 for a in (x, w, dy)]
+    monkeypatch.setenv("AFHIP_NN_X3", "1")
+    out = []
+    for tiny in (0.0, 1e-35, -3e-42):
+        for a, i in zip((x, w, dy), at):
+            a[i] = tiny
+        out.append(_both(af, af.Array(x), af.Array(w), af.Array(dy), g))
+    for o in out[1:]:
+        for a, b in zip(o, out[0]):
+            assert (a != b).mean() < 1e-3
+            np.testing.assert_allclose(a, b, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("scale", [1e-15, 1e-18, 3e-20, 1e-21])
+def test_products_near_the_denormals(af, rng, scale, monkeypatch):
+    # sums from 1e-30 down to a few denormal steps: rounded once, to FP32's
+    # last place or to its smallest step
+    g = ((30, 26, 40, 2), (3, 3, 40, 70), (1, 1), (1, 1), (1, 1))
+    x = (rng.standard_normal(g[0]) * scale).astype(np.float32)
+    w = (rng.standard_normal(g[1]) * scale).astype(np.float32)
+    y64 = oracle.conv2_nn_direct_f64(x, w, *g[2:])
+    dy = (rng.standard_normal(y64.shape) * scale).astype(np.float32)
+    dx64 = oracle.conv2_data_grad_direct_f64(dy, x, w, *g[2:])
+    size = oracle.conv2_nn_direct_f64(abs(x), abs(w), *g[2:]), oracle.conv2_data_grad_direct_f64(abs(dy), x, abs(w), *g[2:])
+    monkeypatch.setenv("AFHIP_NN_X3", "1")
+    for got, ref, s in zip(_both(af, af.Array(x), af.Array(w), af.Array(dy), g), (y64, dx64), size):
+        assert (abs(got - ref) <= 2.0 ** -149 + 5e-7 * s).all()
 
 
 @pytest.mark.parametrize("dims", [(9, 0), (0, 9), (0, 0)], ids=lambda d: "x".join(map(str, d)))
