@@ -278,15 +278,15 @@ static void run_gemm_split(int pass, const ArrayImpl &in, const ArrayImpl &w, af
             pass == 0 ? "convolve2_nn" : "convolve2_gradient_nn");
 }
 
-// FP32 on the BF16 matrix cores in three parts per operand: f32 arrays at
-// their own precision. AFHIP_NN_X3=0 leaves it out, =1 takes it wherever it
+// FP32 on the BF16 matrix cores in three parts per operand: f32 arrays and
+// results at their own precision. AFHIP_NN_X3=0 leaves it out, =1 takes it wherever it
 // serves.
 static int x3_env() {
     const char *e = std::getenv("AFHIP_NN_X3");
     return e && (e[0] == '0' || e[0] == '1') ? e[0] - '0' : -1;
 }
-static bool x3_serves(int pass, const ArrayImpl &in, int precision, const NNGeom &g) {
-    if (in.type != f32 || (precision != AFHIP_PRECISION_DEFAULT && precision != AFHIP_PRECISION_F32)) return false;
+static bool x3_serves(int pass, const ArrayImpl &in, af_dtype out_type, int precision, const NNGeom &g) {
+    if (in.type != f32 || out_type != f32 || (precision != AFHIP_PRECISION_DEFAULT && precision != AFHIP_PRECISION_F32)) return false;
     const char *gather = std::getenv("AFHIP_NN_GATHER");
     if (x3_env() == 0 || (gather && gather[0] == '1')) return false;
     return nn_x3_workspace(pass, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, 1) > 0;
@@ -317,7 +317,7 @@ static std::vector<std::function<void()>> nn_candidates(int pass, const ArrayImp
     if (first) c.push_back(std::move(first));
     const dim4 &o = pass == 0 ? g.y : g.x;
     const long long tiles = (o[2] + 127) / 128 * ((o[0] * o[1] * o[3] + 127) / 128);
-    if (x3_serves(pass, in, precision, g))
+    if (x3_serves(pass, in, out_type, precision, g))
         for (int sp : {1, 2, 4})
             if (sp == 1 || tiles < device_cus()) c.push_back([=, &in, &w, &g] { run_x3(pass, in, w, out, g, sp); });
     for (int sp : kSplitCands)
@@ -339,7 +339,7 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
     const long long need = afhip_k_conv2_nn_patch_workspace(pass, in.type, precision, g.x.d, g.w.d,
                                                             g.y.d, g.st, g.pd, g.dl);
     if (need <= 0) return false;
-    if (x3_env() == 1 && x3_serves(pass, in, precision, g)) {
+    if (x3_env() == 1 && x3_serves(pass, in, out_type, precision, g)) {
         run_x3(pass, in, w, out, g, 1);
         return true;
     }
@@ -368,7 +368,7 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
 // the built-in choice when the autotuner is off.
 static void run_gemm(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype out_type, int precision,
                      void *out, const NNGeom &g, std::function<void()> first = nullptr) {
-    if (x3_env() == 1 && x3_serves(pass, in, precision, g)) {
+    if (x3_env() == 1 && x3_serves(pass, in, out_type, precision, g)) {
         run_x3(pass, in, w, out, g, 1);
         return;
     }
@@ -387,6 +387,15 @@ static af_dtype nn_out_type(af_dtype in, af_dtype requested) {
     return requested;
 }
 
+// Refuses the combinations of storage, arithmetic and result that the kernels
+// refuse, where no kernel runs.
+static void check_nn_types(af_dtype in, af_dtype out, int precision) {
+    ARG_ASSERT(9, precision >= AFHIP_PRECISION_DEFAULT && precision <= AFHIP_PRECISION_F32);
+    const int own = in == afhip_bf16 ? AFHIP_PRECISION_BF16 : AFHIP_PRECISION_F16;
+    if (in != f32 && in != f64 && precision != AFHIP_PRECISION_DEFAULT && precision != own) TYPE_ERROR(1, in);
+    if (out != in && (out != f32 || in == f64)) TYPE_ERROR(10, out);
+}
+
 // cpu::convolve2<T> (NN forward), src/backend/cpu/convolve.cpp:160-167
 static af_array conv2_nn(const ArrayImpl &x, const ArrayImpl &w, const NNGeom &g, int precision,
                          af_dtype out_type) {
@@ -394,6 +403,7 @@ static af_array conv2_nn(const ArrayImpl &x, const ArrayImpl &w, const NNGeom &g
     if (g.y.elements() == 0) return out.release();
     // outputs of padding alone: the kernels read at least one pixel and one tap
     if (g.x.elements() == 0 || g.w.elements() == 0) {
+        check_nn_types(x.type, out_type, precision);
         check_k(afhip_k_fill(out_type, out.data(), 0.0, g.y.elements(), stream()), "fill");
         return out.release();
     }

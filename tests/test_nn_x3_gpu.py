@@ -133,3 +133,22 @@ def test_no_pixels(af, rng, dims, monkeypatch):
         y = af.convolve2NN(X, W, (1, 1), (2, 2), (1, 1))
         assert y.dims == tuple(d + 2 for d in dims) + (70, 2)
         assert not y.to_numpy().any()
+
+
+@pytest.mark.parametrize("f", [3, 7], ids=["patch", "gemm"])
+@pytest.mark.parametrize("env", [None, "AFHIP_NN_X3", "AFHIP_NN_WG"])
+def test_results_of_another_type_are_refused(af, f, env, monkeypatch):
+    # f32 arrays have f32 results; the three-part kernels store nothing else
+    if env:
+        monkeypatch.setenv(env, "1")
+    X, W = af.constant(1, (20, 20, 32, 2)), af.constant(1, (f, f, 32, 64))
+    Y = af.constant(1, (20, 20, 64, 2))
+    geo = ((1, 1), (f // 2, f // 2), (1, 1))
+    for t in (af.f16, af.bf16):
+        for call in (lambda: af.convolve2NN(X, W, *geo, out_type=t),
+                     lambda: af.convolve2NN(af.constant(1, (0, 20, 32, 2)), W, (1, 1), (f, f), out_type=t),
+                     lambda: af.convolve2GradientNN(Y, X, W, Y, *geo, af.AF_CONV_GRADIENT_DATA, out_type=t),
+                     lambda: af.convolve2GradientNN(Y, X, W, Y, *geo, af.AF_CONV_GRADIENT_FILTER, out_type=t)):
+            with pytest.raises(af.AfError) as e:
+                call()
+            assert e.value.code == af.AF_ERR_TYPE
