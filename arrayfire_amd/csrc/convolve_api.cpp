@@ -253,15 +253,26 @@ static std::string nn_key(const char *tag, int pass, const ArrayImpl &in, af_dty
     return k;
 }
 
+struct NNCand {
+    const char *name;
+    int split;
+    std::function<void()> run;
+};
+
 // Index of the variant to run: the autotuner's (timing them now if the key
-// is new), or -1 for the built-in rule.
-static int nn_pick(const std::string &key, const std::vector<std::function<void()>> &cands) {
+// is new), or -1 for the built-in rule. The list depends on more than the
+// layer (switches in the environment, the result's type, the device's CUs), so
+// its names are part of the key: an index is only ever read back for the list
+// it was chosen from.
+static int nn_pick(std::string key, const std::vector<NNCand> &cands) {
     if (cands.size() < 2 || !nn_autotune_on()) return -1;
+    for (size_t i = 0; i < cands.size(); ++i)
+        key += (i ? "," : ":of ") + std::string(cands[i].name) + std::to_string(cands[i].split);
     if (stream_capturing()) {
         const int r = autotune_lookup(key);
         return r >= 0 && r < (int)cands.size() ? r : -1;
     }
-    return autotune_pick(key, (int)cands.size(), [&](int c) { cands[c](); });
+    return autotune_pick(key, (int)cands.size(), [&](int c) { cands[c].run(); });
 }
 
 static const int kSplitCands[] = {1, 2, 4, 8, 16};
@@ -310,19 +321,20 @@ static void run_patch_kernels(int pass, const ArrayImpl &in, const ArrayImpl &w,
 // Candidates: `first` (the patch kernels or the polyphase split, where they
 // serve), then the GEMM with the split counts worth a try. Splitting pays
 // only where the GEMM's own tiles leave CUs idle.
-static std::vector<std::function<void()>> nn_candidates(int pass, const ArrayImpl &in, const ArrayImpl &w,
-                                                        af_dtype out_type, int precision, void *out,
-                                                        const NNGeom &g, std::function<void()> first) {
-    std::vector<std::function<void()>> c;
-    if (first) c.push_back(std::move(first));
+static std::vector<NNCand> nn_candidates(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype out_type,
+                                         int precision, void *out, const NNGeom &g, const char *first_name,
+                                         std::function<void()> first) {
+    std::vector<NNCand> c;
+    if (first) c.push_back({first_name, 1, std::move(first)});
     const dim4 &o = pass == 0 ? g.y : g.x;
     const long long tiles = (o[2] + 127) / 128 * ((o[0] * o[1] * o[3] + 127) / 128);
     if (x3_serves(pass, in, out_type, precision, g))
         for (int sp : {1, 2, 4})
-            if (sp == 1 || tiles < device_cus()) c.push_back([=, &in, &w, &g] { run_x3(pass, in, w, out, g, sp); });
+            if (sp == 1 || tiles < device_cus())
+                c.push_back({"x3/", sp, [=, &in, &w, &g] { run_x3(pass, in, w, out, g, sp); }});
     for (int sp : kSplitCands)
         if (sp == 1 || tiles < device_cus())
-            c.push_back([=, &in, &w, &g] { run_gemm_split(pass, in, w, out_type, precision, out, g, sp); });
+            c.push_back({"gemm/", sp, [=, &in, &w, &g] { run_gemm_split(pass, in, w, out_type, precision, out, g, sp); }});
     return c;
 }
 
@@ -349,7 +361,7 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
         patch();
         return true;
     }
-    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, patch);
+    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, "patch/", patch);
     int c = nn_pick(nn_key("nn3", pass, in, out_type, precision, g), cands);
     if (c < 0) {
         const long long tiles = afhip_k_conv2_nn_patch_tiles(pass, in.type, precision, g.x.d, g.w.d, g.y.d, g.st,
@@ -357,7 +369,7 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
         c = tiles * 4 >= device_cus() ? 0 : -1;
     }
     if (c >= 0)
-        cands[c]();
+        cands[c].run();
     else
         run_gemm_split(pass, in, w, out_type, precision, out, g, 0);
     return true;
@@ -373,11 +385,11 @@ static void run_gemm(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype
         return;
     }
     const bool has_first = (bool)first;
-    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, std::move(first));
+    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, "poly/", std::move(first));
     int c = nn_pick(nn_key("nn_gemm3", pass, in, out_type, precision, g), cands);
     if (c < 0 && has_first) c = 0;
     if (c >= 0)
-        cands[c]();
+        cands[c].run();
     else
         run_gemm_split(pass, in, w, out_type, precision, out, g, 0);
 }
@@ -511,11 +523,14 @@ static void run_wgrad(const ArrayImpl &dy, const ArrayImpl &x, const NNGeom &g, 
         gemm(2 * cus);
         return;
     }
-    std::vector<std::function<void()>> cands{old, [&] { gemm(cus); }, [&] { gemm(2 * cus); }, [&] { gemm(4 * cus); }};
+    const std::vector<NNCand> cands{{"rows/", 1, old},
+                                    {"wgemm/", 1, [&] { gemm(cus); }},
+                                    {"wgemm/", 2, [&] { gemm(2 * cus); }},
+                                    {"wgemm/", 4, [&] { gemm(4 * cus); }}};
     int c = nn_pick(nn_key("nn_wg", 2, x, out_type, precision, g), cands);
     if (c < 0)
         c = afhip_k_conv2_nn_wgrad_rows_workspace(x.type, precision, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl) > 0 ? 0 : 2;
-    cands[c]();
+    cands[c].run();
 }
 
 // cpu::conv2FilterGradient<T>, src/backend/cpu/convolve.cpp:213-243

@@ -4,6 +4,8 @@ import sys
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+# choices timed under the tests' switches stay out of the user's file
+os.environ.setdefault("AFHIP_AUTOTUNE_CACHE", "off")
 if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
