@@ -214,13 +214,17 @@ static int device_cus() {
     return n;
 }
 
-// ---- NN variant choice. The autotuner (autotune.cpp) times the candidate
-// variants (the patch kernels or the polyphase split where they serve; the
-// GEMM, with splits of the reduction where its tiles leave CUs idle) on the
-// first call of a geometry and caches the fastest under a key of (pass,
-// dtypes, precision, dims, stride, padding, dilation). Under stream capture
-// only cached choices are used. AFHIP_NN_AUTOTUNE=0 (or an explicit
-// AFHIP_NN_SPLIT) keeps the built-in rules.
+// ---- NN variant choice. Layers that fill the chip with the patch kernels'
+// tiles, strided data gradients that fill it phase by phase and all filter
+// gradients go by rules on the sizes (patch_by_rule, rows_by_rule): no timing on
+// the first call, and the same kernel, so the same bits, on every run. The other
+// forward passes and data gradients are the autotuner's (autotune.cpp): it times
+// the candidate variants (the patch kernels where they serve; the GEMM with
+// splits of the reduction) on the first call of a geometry and caches the
+// fastest under a key of (pass, dtypes, precision, dims, stride, padding,
+// dilation). Under stream capture only cached choices are used.
+// AFHIP_NN_AUTOTUNE=0 (or an explicit AFHIP_NN_SPLIT) keeps built-in rules there
+// too.
 static bool nn_autotune_on() {
     const char *a = std::getenv("AFHIP_NN_AUTOTUNE");
     const char *sp = std::getenv("AFHIP_NN_SPLIT");
@@ -318,14 +322,14 @@ static void run_patch_kernels(int pass, const ArrayImpl &in, const ArrayImpl &w,
             pass == 0 ? "convolve2_nn" : "convolve2_gradient_nn");
 }
 
-// Candidates: `first` (the patch kernels or the polyphase split, where they
-// serve), then the GEMM with the split counts worth a try. Splitting pays
-// only where the GEMM's own tiles leave CUs idle.
+// Candidates: the patch kernels, where they serve, then the GEMM with the split
+// counts worth a try. Splitting pays only where the GEMM's own tiles leave CUs
+// idle.
 static std::vector<NNCand> nn_candidates(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype out_type,
-                                         int precision, void *out, const NNGeom &g, const char *first_name,
-                                         std::function<void()> first) {
+                                         int precision, void *out, const NNGeom &g,
+                                         std::function<void()> patch) {
     std::vector<NNCand> c;
-    if (first) c.push_back({first_name, 1, std::move(first)});
+    if (patch) c.push_back({"patch/", 1, std::move(patch)});
     const dim4 &o = pass == 0 ? g.y : g.x;
     const long long tiles = (o[2] + 127) / 128 * ((o[0] * o[1] * o[3] + 127) / 128);
     if (x3_serves(pass, in, out_type, precision, g))
@@ -338,12 +342,46 @@ static std::vector<NNCand> nn_candidates(int pass, const ArrayImpl &in, const Ar
     return c;
 }
 
-// The autotuned choice between the patch kernels and the GEMM: neither wins by
-// a rule that the shape alone gives (BF16 56x56x64x32 -> 128: 28 us on the
-// weights-resident kernel, 42 us on the GEMM; 28x28x128x32 -> 128, whose rows
-// are no whole 16-byte vectors: 55 and 24; 79x79x3x32 -> 32: 34 and 43).
-// Built-in rule: the patch kernels when they launch at least a quarter of the
-// CUs' workgroups. AFHIP_NN_SMALL=0 keeps every served layer on them.
+// Whether the GEMM reads channel-last copies (operands at their own precision,
+// copies within its offsets) rather than single elements.
+static bool gemm_copies(int pass, const ArrayImpl &in, int precision, const NNGeom &g) {
+    return afhip_k_conv2_nn_gemm_split_workspace(pass, in.type, precision, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, 1) > 0;
+}
+
+// Whether the rows of x and y are whole vectors of 16 bytes.
+static bool whole_rows(const NNGeom &g, af_dtype t) {
+    const dim_t v = t == f32 ? 4 : 8;
+    return g.x[0] % v == 0 && g.y[0] % v == 0;
+}
+
+// Of the layers whose patch tiles fill the chip, those that the patch kernels
+// run faster than the GEMM (x3 for f32), us:
+//  * f32: 9 to 16 reduction channels, one chunk of the patch kernels and half of
+//    a GEMM slice (60x60x16x32 -> 16, 3x3: 31 and 43), and 1x1 filters that do
+//    not widen the channels, where the copies cost as much as the product
+//    (64x64x128x32 -> 128: 63 and 74; to 256 from 56x56x64x32: 73 and 58). Else
+//    the GEMM (28x28x128x64 -> 128, 3x3: 171 and 121; 62x62x128x16 -> 128: 189
+//    and 145);
+//  * 16-bit: few channels (57x57x3x64 -> 64, 3x3: 37 and 44), and whole rows
+//    under the weights-resident kernel or under pipelined stages that do not
+//    widen the channels (56x56x64x32 -> 128, 3x3: 29 and 39; 64x64x128x32 ->
+//    128, 1x1: 29 and 32; 32x32x96x64 -> 96, 5x5: 57 and 64). Else the GEMM
+//    (28x28x128x64 -> 128: 77 and 37; 48x48x64x64 -> 32, 5x5: 83 and 71;
+//    96x96x64x32 -> 64, 5x5, stride 2: 178 and 53; rows of 8 pixels 269 and
+//    110).
+static bool patch_by_rule(int pass, const ArrayImpl &in, const NNGeom &g) {
+    const dim_t R = pass == 0 ? g.x[2] : g.w[3], M = pass == 0 ? g.w[3] : g.x[2], taps = g.w[0] * g.w[1];
+    const bool whole = whole_rows(g, in.type), unit = g.st[0] == 1 && g.st[1] == 1;
+    if (in.type == f32) return whole && ((R > 8 && R <= 16) || (taps == 1 && R >= M));
+    if (R <= 16) return true;
+    if (!whole || g.x[0] < 16) return false;
+    if (taps == 1) return unit && R >= M;
+    return taps <= 9 ? unit || taps == 9 : unit && R >= 96;
+}
+
+// AFHIP_NN_SMALL=0 keeps every served layer on the patch kernels. Built-in rule
+// for the autotuned layers: the patch kernels when they launch at least a
+// quarter of the CUs' workgroups.
 static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype out_type,
                       int precision, void *out, const NNGeom &g) {
     const char *env = std::getenv("AFHIP_NN_GATHER");
@@ -351,7 +389,8 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
     const long long need = afhip_k_conv2_nn_patch_workspace(pass, in.type, precision, g.x.d, g.w.d,
                                                             g.y.d, g.st, g.pd, g.dl);
     if (need <= 0) return false;
-    if (x3_env() == 1 && x3_serves(pass, in, out_type, precision, g)) {
+    const bool x3 = x3_serves(pass, in, out_type, precision, g);
+    if (x3_env() == 1 && x3) {
         run_x3(pass, in, w, out, g, 1);
         return true;
     }
@@ -361,13 +400,21 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
         patch();
         return true;
     }
-    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, "patch/", patch);
-    int c = nn_pick(nn_key("nn3", pass, in, out_type, precision, g), cands);
-    if (c < 0) {
-        const long long tiles = afhip_k_conv2_nn_patch_tiles(pass, in.type, precision, g.x.d, g.w.d, g.y.d, g.st,
-                                                             g.pd, g.dl);
-        c = tiles * 4 >= device_cus() ? 0 : -1;
+    const long long tiles = afhip_k_conv2_nn_patch_tiles(pass, in.type, precision, g.x.d, g.w.d, g.y.d, g.st, g.pd,
+                                                         g.dl);
+    if (tiles >= device_cus()) {
+        const bool gemm = in.type == f32 ? x3 : gemm_copies(pass, in, precision, g);
+        if (!gemm || patch_by_rule(pass, in, g))
+            patch();
+        else if (x3)
+            run_x3(pass, in, w, out, g, 1);
+        else
+            run_gemm_split(pass, in, w, out_type, precision, out, g, 1);
+        return true;
     }
+    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, patch);
+    int c = nn_pick(nn_key("nn3", pass, in, out_type, precision, g), cands);
+    if (c < 0) c = tiles * 4 >= device_cus() ? 0 : -1;
     if (c >= 0)
         cands[c].run();
     else
@@ -376,18 +423,15 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
 }
 
 // The GEMM for every other geometry, its split count autotuned (built-in
-// rule: split when that fills the chip); `first`: another kernel that serves,
-// the built-in choice when the autotuner is off.
+// rule: split when that fills the chip).
 static void run_gemm(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype out_type, int precision,
-                     void *out, const NNGeom &g, std::function<void()> first = nullptr) {
+                     void *out, const NNGeom &g) {
     if (x3_env() == 1 && x3_serves(pass, in, out_type, precision, g)) {
         run_x3(pass, in, w, out, g, 1);
         return;
     }
-    const bool has_first = (bool)first;
-    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, "poly/", std::move(first));
-    int c = nn_pick(nn_key("nn_gemm3", pass, in, out_type, precision, g), cands);
-    if (c < 0 && has_first) c = 0;
+    const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, nullptr);
+    const int c = nn_pick(nn_key("nn_gemm3", pass, in, out_type, precision, g), cands);
     if (c >= 0)
         cands[c].run();
     else
@@ -447,23 +491,30 @@ static af_array conv2_data_grad(const ArrayImpl &dy, const ArrayImpl &x, const A
         return out.release();
     }
     if (run_patch(1, dy, w, out_type, precision, o, g)) return out.release();
-    // strided layers: the autotuned choice between the polyphase split into
-    // stride-1 convolutions on the patch kernels, when its phases fill the
-    // chip, and the GEMM over phase-ordered pixels (AFHIP_NN_GATHER=1 keeps
-    // the GEMM)
-    const char *gather = std::getenv("AFHIP_NN_GATHER");
-    if (!(gather && gather[0] == '1')) {
-        const long long pb = afhip_k_conv2_nn_dgrad_poly_workspace(x.type, out_type, precision, g.x.d, g.w.d,
-                                                                  g.y.d, g.st, g.pd, g.dl);
-        if (pb > 0) {
-            run_gemm(1, dy, w, out_type, precision, o, g, [&] {
-                auto ws = scratch((size_t)pb);
-                check_k(afhip_k_conv2_nn_dgrad_poly(x.type, out_type, precision, o, dy.data(), w.data(), g.x.d,
-                                                    g.w.d, g.y.d, g.st, g.pd, g.dl, ws->ptr, pb, stream()),
-                        "convolve2_gradient_nn");
-            });
-            return out.release();
+    // Strided layers whose phases fill the chip: the GEMM over phase-ordered
+    // pixels where it reads channel-last copies (57x57x64x64 -> 128, 3x3, stride
+    // 2: BF16 58 us, FP32 104 us; 302 and 349 us as polyphase stride-1
+    // convolutions on the patch kernels, which need a launch per phase to pack,
+    // convolve and scatter), the polyphase split elsewhere. AFHIP_NN_POLY=1 takes
+    // the split, AFHIP_NN_GATHER=1 leaves it out.
+    const char *gather = std::getenv("AFHIP_NN_GATHER"), *pe = std::getenv("AFHIP_NN_POLY");
+    const long long pb = gather && gather[0] == '1'
+                             ? 0
+                             : afhip_k_conv2_nn_dgrad_poly_workspace(x.type, out_type, precision, g.x.d, g.w.d, g.y.d,
+                                                                     g.st, g.pd, g.dl);
+    if (pb > 0) {
+        const bool poly = pe && pe[0] == '1';
+        if (!poly && x3_serves(1, dy, out_type, precision, g)) {
+            run_x3(1, dy, w, o, g, 1);
+        } else if (!poly && gemm_copies(1, dy, precision, g)) {
+            run_gemm_split(1, dy, w, out_type, precision, o, g, 1);
+        } else {
+            auto ws = scratch((size_t)pb);
+            check_k(afhip_k_conv2_nn_dgrad_poly(x.type, out_type, precision, o, dy.data(), w.data(), g.x.d, g.w.d,
+                                                g.y.d, g.st, g.pd, g.dl, ws->ptr, pb, stream()),
+                    "convolve2_gradient_nn");
         }
+        return out.release();
     }
     run_gemm(1, dy, w, out_type, precision, o, g);
     return out.release();
@@ -491,12 +542,25 @@ static void wgrad_rows_or_gather(const ArrayImpl &dy, const ArrayImpl &x, const 
             "convolve2_gradient_nn");
 }
 
-// The autotuned choice between those and the channel-last GEMM with about one,
-// two or four workgroups per CU (56x56x64x32 -> 128, 3x3, BF16: rows 45 us,
-// GEMM 43; 60x60x16x32 -> 16: 52 and 31; 27x27x96x16 -> 128, 5x5: gather 186, GEMM
-// 37). Built-in rule: the
-// row-staged kernels where they serve, else the GEMM. AFHIP_NN_WG=0 leaves the
-// GEMM out, =1 takes it wherever it serves.
+// Of the filter gradients that the row-staged kernels serve, those that they run
+// faster than the GEMM over channel-last copies, us: whole rows, and
+//  * f32: large 1x1 layers of one tile (56x56x64x32 -> 64: 41 and 45;
+//    112x112x64x8 -> 64: 38 and 45). Else the GEMM (56x56x64x32 -> 128, 3x3: 205
+//    and 124; 41x67x16x30 -> 16, 1x1: 50 and 32);
+//  * 16-bit: rows of 16 pixels and more and a full tile of filters or channels,
+//    unless the other side is a few channels of very many pixels (56x56x64x32 ->
+//    128, 3x3: 42 and 49; 64x64x64x64 -> 64: 46 and 64). Else the GEMM
+//    (56x56x16x32 -> 16: 36 and 29; 8x8x256x128 -> 256: 61 and 40; 28x28x128x32
+//    -> 128: 72 and 33; 224x224x3x8 -> 64: 94 and 81).
+static bool rows_by_rule(const ArrayImpl &x, const NNGeom &g) {
+    if (!whole_rows(g, x.type)) return false;
+    const dim_t lo = std::min(g.x[2], g.w[3]), hi = std::max(g.x[2], g.w[3]), px = g.y[0] * g.y[1] * g.y[3];
+    if (x.type == f32) return g.w[0] * g.w[1] == 1 && hi <= 64 && px >= 65536;
+    return g.x[0] >= 16 && hi >= 64 && (lo >= 16 || px < 250000);
+}
+
+// By that rule, for any other geometry the GEMM. AFHIP_NN_WG=0 leaves the GEMM
+// out, =1 takes it wherever it serves.
 static void run_wgrad(const ArrayImpl &dy, const ArrayImpl &x, const NNGeom &g, int precision, af_dtype out_type,
                       void *o) {
     const char *env = std::getenv("AFHIP_NN_GATHER"), *wg = std::getenv("AFHIP_NN_WG");
@@ -505,32 +569,22 @@ static void run_wgrad(const ArrayImpl &dy, const ArrayImpl &x, const NNGeom &g, 
                      precision == (x.type == f32   ? AFHIP_PRECISION_F32
                                    : x.type == f16 ? AFHIP_PRECISION_F16
                                                    : AFHIP_PRECISION_BF16);
-    auto old = [&] { wgrad_rows_or_gather(dy, x, g, precision, out_type, o, gather); };
-    auto gemm = [&](int target) {
-        const long long need = nn_wgemm_workspace(x.type, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, target);
-        auto ws = scratch((size_t)need);
-        check_k(nn_wgemm(x.type, out_type, o, x.data(), dy.data(), g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, target,
-                         ws->ptr, need, stream()),
-                "convolve2_gradient_nn");
-    };
-    const int cus = device_cus();
-    if (gather || !own || (wg && wg[0] == '0') ||
-        nn_wgemm_workspace(x.type, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, cus) <= 0) {
-        old();
+    // two workgroups per CU
+    const int target = 2 * device_cus();
+    const long long need = gather || !own || (wg && wg[0] == '0')
+                               ? 0
+                               : nn_wgemm_workspace(x.type, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, target);
+    const bool rows = need <= 0 || (!(wg && wg[0] == '1') && rows_by_rule(x, g) &&
+                                    afhip_k_conv2_nn_wgrad_rows_workspace(x.type, precision, g.x.d, g.w.d, g.y.d, g.st,
+                                                                          g.pd, g.dl) > 0);
+    if (rows) {
+        wgrad_rows_or_gather(dy, x, g, precision, out_type, o, gather);
         return;
     }
-    if (wg && wg[0] == '1') {
-        gemm(2 * cus);
-        return;
-    }
-    const std::vector<NNCand> cands{{"rows/", 1, old},
-                                    {"wgemm/", 1, [&] { gemm(cus); }},
-                                    {"wgemm/", 2, [&] { gemm(2 * cus); }},
-                                    {"wgemm/", 4, [&] { gemm(4 * cus); }}};
-    int c = nn_pick(nn_key("nn_wg", 2, x, out_type, precision, g), cands);
-    if (c < 0)
-        c = afhip_k_conv2_nn_wgrad_rows_workspace(x.type, precision, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl) > 0 ? 0 : 2;
-    cands[c].run();
+    auto ws = scratch((size_t)need);
+    check_k(nn_wgemm(x.type, out_type, o, x.data(), dy.data(), g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, target, ws->ptr,
+                     need, stream()),
+            "convolve2_gradient_nn");
 }
 
 // cpu::conv2FilterGradient<T>, src/backend/cpu/convolve.cpp:213-243

@@ -1,7 +1,7 @@
 // Filter gradient from channel-last copies (kernels/nn_wgemm.hip), any
 // geometry: bf16 and f16 arrays at their own precision, f32 arrays in three
-// BF16 parts per operand. type: af_dtype of x and dy; target: workgroups to
-// aim for (the split of the pixels follows from it).
+// BF16 parts per operand. type: af_dtype of x and dy; target: the most
+// workgroups to split the pixels into.
 #pragma once
 #include <hip/hip_runtime.h>
 
