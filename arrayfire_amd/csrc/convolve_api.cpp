@@ -362,7 +362,8 @@ static bool whole_rows(const NNGeom &g, af_dtype t) {
 //    (64x64x128x32 -> 128: 63 and 74; to 256 from 56x56x64x32: 73 and 58). Else
 //    the GEMM (28x28x128x64 -> 128, 3x3: 171 and 121; 62x62x128x16 -> 128: 189
 //    and 145);
-//  * 16-bit: few channels (57x57x3x64 -> 64, 3x3: 37 and 44), and whole rows
+//  * 16-bit: few channels (57x57x3x64 -> 64, 3x3: 37 and 44; to more than 32
+//    over odd rows the GEMM, 68x35x16x27 -> 128: 27 and 22), and whole rows
 //    under the weights-resident kernel or under pipelined stages that do not
 //    widen the channels (56x56x64x32 -> 128, 3x3: 29 and 39; 64x64x128x32 ->
 //    128, 1x1: 29 and 32; 32x32x96x64 -> 96, 5x5: 57 and 64). Else the GEMM
@@ -373,7 +374,7 @@ static bool patch_by_rule(int pass, const ArrayImpl &in, const NNGeom &g) {
     const dim_t R = pass == 0 ? g.x[2] : g.w[3], M = pass == 0 ? g.w[3] : g.x[2], taps = g.w[0] * g.w[1];
     const bool whole = whole_rows(g, in.type), unit = g.st[0] == 1 && g.st[1] == 1;
     if (in.type == f32) return whole && ((R > 8 && R <= 16) || (taps == 1 && R >= M));
-    if (R <= 16) return true;
+    if (R <= 8 || (R <= 16 && (whole || M <= 32))) return true;
     if (!whole || g.x[0] < 16) return false;
     if (taps == 1) return unit && R >= M;
     return taps <= 9 ? unit || taps == 9 : unit && R >= 96;
@@ -543,20 +544,24 @@ static void wgrad_rows_or_gather(const ArrayImpl &dy, const ArrayImpl &x, const 
 }
 
 // Of the filter gradients that the row-staged kernels serve, those that they run
-// faster than the GEMM over channel-last copies, us: whole rows, and
-//  * f32: large 1x1 layers of one tile (56x56x64x32 -> 64: 41 and 45;
-//    112x112x64x8 -> 64: 38 and 45). Else the GEMM (56x56x64x32 -> 128, 3x3: 205
-//    and 124; 41x67x16x30 -> 16, 1x1: 50 and 32);
-//  * 16-bit: rows of 16 pixels and more and a full tile of filters or channels,
-//    unless the other side is a few channels of very many pixels (56x56x64x32 ->
-//    128, 3x3: 42 and 49; 64x64x64x64 -> 64: 46 and 64). Else the GEMM
-//    (56x56x16x32 -> 16: 36 and 29; 8x8x256x128 -> 256: 61 and 40; 28x28x128x32
-//    -> 128: 72 and 33; 224x224x3x8 -> 64: 94 and 81).
+// faster than the GEMM over channel-last copies, us: many whole rows, and
+//  * f32: 1x1 filters of one tile (56x56x64x32 -> 64: 41 and 45; 112x112x64x8 ->
+//    64: 38 and 45). Else the GEMM (56x56x64x32 -> 128, 3x3: 205 and 124;
+//    41x67x16x30 -> 16, 1x1: 50 and 32);
+//  * 16-bit: rows that fill four fifths of the kernels' 32-pixel steps, with
+//    a full tile of filters or channels and a quarter of one of the other, and
+//    1x1 filters of few tiles (56x56x64x32 -> 128, 3x3: 42 and 49; 64x64x64x64
+//    -> 64: 46 and 64; 32x32x256x32 -> 64, 1x1: 19 and 25). Else the GEMM
+//    (40x40x64x32 -> 64: 34 and 27; 56x56x16x32 -> 16: 36 and 29; 72x72x3x32 ->
+//    64: 53 and 46; 28x28x128x32 -> 128: 72 and 33; 72x70x48x3 -> 256: 35 and
+//    28; 80x80x256x4 -> 256, 1x1: 42 and 29).
 static bool rows_by_rule(const ArrayImpl &x, const NNGeom &g) {
     if (!whole_rows(g, x.type)) return false;
     const dim_t lo = std::min(g.x[2], g.w[3]), hi = std::max(g.x[2], g.w[3]), px = g.y[0] * g.y[1] * g.y[3];
-    if (x.type == f32) return g.w[0] * g.w[1] == 1 && hi <= 64 && px >= 65536;
-    return g.x[0] >= 16 && hi >= 64 && (lo >= 16 || px < 250000);
+    const dim_t taps = g.w[0] * g.w[1], ow = g.y[0];
+    if (x.type == f32) return taps == 1 && hi <= 64 && px >= 65536;
+    return px >= 32768 && hi >= 64 && lo >= 16 && ow >= 32 && ow * 5 >= (ow + 31) / 32 * 32 * 4 &&
+           (taps > 1 || lo * hi * g.st[0] * g.st[1] <= 16384);
 }
 
 // By that rule, for any other geometry the GEMM. AFHIP_NN_WG=0 leaves the GEMM
@@ -569,11 +574,10 @@ static void run_wgrad(const ArrayImpl &dy, const ArrayImpl &x, const NNGeom &g, 
                      precision == (x.type == f32   ? AFHIP_PRECISION_F32
                                    : x.type == f16 ? AFHIP_PRECISION_F16
                                                    : AFHIP_PRECISION_BF16);
-    // two workgroups per CU
-    const int target = 2 * device_cus();
+    const int cus = device_cus();
     const long long need = gather || !own || (wg && wg[0] == '0')
                                ? 0
-                               : nn_wgemm_workspace(x.type, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, target);
+                               : nn_wgemm_workspace(x.type, g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, cus);
     const bool rows = need <= 0 || (!(wg && wg[0] == '1') && rows_by_rule(x, g) &&
                                     afhip_k_conv2_nn_wgrad_rows_workspace(x.type, precision, g.x.d, g.w.d, g.y.d, g.st,
                                                                           g.pd, g.dl) > 0);
@@ -582,7 +586,7 @@ static void run_wgrad(const ArrayImpl &dy, const ArrayImpl &x, const NNGeom &g, 
         return;
     }
     auto ws = scratch((size_t)need);
-    check_k(nn_wgemm(x.type, out_type, o, x.data(), dy.data(), g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, target, ws->ptr,
+    check_k(nn_wgemm(x.type, out_type, o, x.data(), dy.data(), g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, cus, ws->ptr,
                      need, stream()),
             "convolve2_gradient_nn");
 }

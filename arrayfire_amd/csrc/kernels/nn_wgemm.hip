@@ -364,10 +364,10 @@ struct WgLayout {
     long long off_d = 0, off_flag = 0, off_part = 0, total = 0;
 };
 static bool wg_setup(int type, const long long *xd, const long long *wd, const long long *yd, const long long *st,
-                     const long long *pd, const long long *dl, int target, WgParams *p, WgLayout *L, int *tt) {
+                     const long long *pd, const long long *dl, int cus, WgParams *p, WgLayout *L, int *tt) {
     const bool x3 = type == DT_F32;
     if (!x3 && type != DT_BF16 && type != DT_F16) return false;
-    if (wd[2] != xd[2] || yd[2] != wd[3] || yd[3] != xd[3] || target < 1) return false;
+    if (wd[2] != xd[2] || yd[2] != wd[3] || yd[3] != xd[3] || cus < 1) return false;
     for (int i = 0; i < 2; ++i)
         if (st[i] < 1 || dl[i] < 1) return false;
     const long long npx = xd[0] * xd[1] * xd[3], npd = yd[0] * yd[1] * yd[3], lim = 1LL << 30;  // offsets past a resource's end must not wrap
@@ -413,9 +413,13 @@ static bool wg_setup(int type, const long long *xd, const long long *wd, const l
     if (ntile >= (1LL << 24)) return false;
     p->ntile = (int)ntile;
     p->slices = (int)((npd + 31) / 32);
-    // as many splits as fit the target, and not one more: 28x28x128x64 -> 128,
-    // 3x3, FP32, two workgroups per CU: 42 splits (504 of 512) 113 us, 43 (516) 157
-    long long split = std::max<long long>(1, target / ntile);
+    // As many splits as two workgroups per CU hold, and not one more:
+    // 28x28x128x64 -> 128, 3x3, FP32: 42 splits (504 of 512) 113 us, 43 (516) 157.
+    // The 16-bit kernels, of which four fit, take twice as many where each has
+    // pixels enough (32x32x96x64 -> 96, 5x5: 97 us against 110; 28x28x128x64 ->
+    // 128, with 37 slices each of the larger share: 50 against 49).
+    const long long wide = !x3 && p->slices * ntile > 112LL * cus ? 4 : 2;
+    long long split = std::max<long long>(1, wide * cus / ntile);
     const long long each = (long long)p->RS * p->K * p->C * 4;
     split = std::min<long long>(split, (p->slices + 4 * SL - 1) / (4 * SL));  // at least four stages each
     split = std::max<long long>(1, std::min<long long>(split, (256LL << 20) / each));
@@ -432,20 +436,20 @@ static bool wg_setup(int type, const long long *xd, const long long *wd, const l
 }
 
 long long nn_wgemm_workspace(int type, const long long *xd, const long long *wd, const long long *yd,
-                             const long long *st, const long long *pd, const long long *dl, int target) {
+                             const long long *st, const long long *pd, const long long *dl, int cus) {
     WgParams p;
     WgLayout L;
     int tt;
-    return wg_setup(type, xd, wd, yd, st, pd, dl, target, &p, &L, &tt) ? L.total : 0;
+    return wg_setup(type, xd, wd, yd, st, pd, dl, cus, &p, &L, &tt) ? L.total : 0;
 }
 
 int nn_wgemm(int type, int out_type, void *dw, const void *x, const void *dy, const long long *xd, const long long *wd,
-             const long long *yd, const long long *st, const long long *pd, const long long *dl, int target, void *ws,
+             const long long *yd, const long long *st, const long long *pd, const long long *dl, int cus, void *ws,
              long long ws_bytes, hipStream_t s) {
     WgParams p;
     WgLayout L;
     int tt;
-    if (!wg_setup(type, xd, wd, yd, st, pd, dl, target, &p, &L, &tt)) return K_ERR_NOT_SUPPORTED;
+    if (!wg_setup(type, xd, wd, yd, st, pd, dl, cus, &p, &L, &tt)) return K_ERR_NOT_SUPPORTED;
     if (out_type != DT_F32 && out_type != type) return K_ERR_TYPE;
     if (ws == nullptr || ws_bytes < L.total) return K_ERR_ARG;
     char *xc = (char *)ws, *dc = xc + L.off_d;
