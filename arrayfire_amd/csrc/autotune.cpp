@@ -104,7 +104,13 @@ int autotune_pick(const std::string &key, int ncand, const std::function<void(in
     // fastest of three trials of three launches, so that one disturbed trial
     // does not decide the choice.
     for (int c = 0; c < ncand; ++c) {
-        launch(c);
+        try {
+            launch(c);
+        } catch (const AfError &e) {
+            // a workspace that does not fit: not a candidate, unless nothing is
+            if (e.code() != AF_ERR_NO_MEM || (c == ncand - 1 && best_ms == 1e30f)) throw;
+            continue;
+        }
         float cand_ms = 1e30f;
         for (int trial = 0; trial < 3; ++trial) {
             check_hip(hipEventRecord(e0, s), "hipEventRecord");

@@ -342,6 +342,19 @@ static std::vector<NNCand> nn_candidates(int pass, const ArrayImpl &in, const Ar
     return c;
 }
 
+// first, or second where the device has no room for first's workspace: copies
+// of both operands, up to 2 GiB each, where the kernels that do without need
+// the packed weights or nothing. Workspaces are allocated before any launch.
+template <typename A, typename B>
+static void or_with_less_memory(A &&first, B &&second) {
+    try {
+        first();
+    } catch (const AfError &e) {
+        if (e.code() != AF_ERR_NO_MEM) throw;
+        second();
+    }
+}
+
 // Whether the GEMM reads channel-last copies (operands at their own precision,
 // copies within its offsets) rather than single elements.
 static bool gemm_copies(int pass, const ArrayImpl &in, int precision, const NNGeom &g) {
@@ -408,16 +421,16 @@ static bool run_patch(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtyp
         if (!gemm || patch_by_rule(pass, in, g))
             patch();
         else if (x3)
-            run_x3(pass, in, w, out, g, 1);
+            or_with_less_memory([&] { run_x3(pass, in, w, out, g, 1); }, patch);
         else
-            run_gemm_split(pass, in, w, out_type, precision, out, g, 1);
+            or_with_less_memory([&] { run_gemm_split(pass, in, w, out_type, precision, out, g, 1); }, patch);
         return true;
     }
     const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, patch);
     int c = nn_pick(nn_key("nn3", pass, in, out_type, precision, g), cands);
     if (c < 0) c = tiles * 4 >= device_cus() ? 0 : -1;
     if (c >= 0)
-        cands[c].run();
+        or_with_less_memory(cands[c].run, patch);
     else
         run_gemm_split(pass, in, w, out_type, precision, out, g, 0);
     return true;
@@ -434,7 +447,7 @@ static void run_gemm(int pass, const ArrayImpl &in, const ArrayImpl &w, af_dtype
     const auto cands = nn_candidates(pass, in, w, out_type, precision, out, g, nullptr);
     const int c = nn_pick(nn_key("nn_gemm3", pass, in, out_type, precision, g), cands);
     if (c >= 0)
-        cands[c].run();
+        or_with_less_memory(cands[c].run, [&] { run_gemm_split(pass, in, w, out_type, precision, out, g, 1); });
     else
         run_gemm_split(pass, in, w, out_type, precision, out, g, 0);
 }
@@ -504,17 +517,19 @@ static af_array conv2_data_grad(const ArrayImpl &dy, const ArrayImpl &x, const A
                              : afhip_k_conv2_nn_dgrad_poly_workspace(x.type, out_type, precision, g.x.d, g.w.d, g.y.d,
                                                                      g.st, g.pd, g.dl);
     if (pb > 0) {
-        const bool poly = pe && pe[0] == '1';
-        if (!poly && x3_serves(1, dy, out_type, precision, g)) {
-            run_x3(1, dy, w, o, g, 1);
-        } else if (!poly && gemm_copies(1, dy, precision, g)) {
-            run_gemm_split(1, dy, w, out_type, precision, o, g, 1);
-        } else {
+        const auto poly = [&] {
             auto ws = scratch((size_t)pb);
             check_k(afhip_k_conv2_nn_dgrad_poly(x.type, out_type, precision, o, dy.data(), w.data(), g.x.d, g.w.d,
                                                 g.y.d, g.st, g.pd, g.dl, ws->ptr, pb, stream()),
                     "convolve2_gradient_nn");
-        }
+        };
+        const bool gemm = !(pe && pe[0] == '1');
+        if (gemm && x3_serves(1, dy, out_type, precision, g))
+            or_with_less_memory([&] { run_x3(1, dy, w, o, g, 1); }, poly);
+        else if (gemm && gemm_copies(1, dy, precision, g))
+            or_with_less_memory([&] { run_gemm_split(1, dy, w, out_type, precision, o, g, 1); }, poly);
+        else
+            poly();
         return out.release();
     }
     run_gemm(1, dy, w, out_type, precision, o, g);
@@ -581,14 +596,19 @@ static void run_wgrad(const ArrayImpl &dy, const ArrayImpl &x, const NNGeom &g, 
     const bool rows = need <= 0 || (!(wg && wg[0] == '1') && rows_by_rule(x, g) &&
                                     afhip_k_conv2_nn_wgrad_rows_workspace(x.type, precision, g.x.d, g.w.d, g.y.d, g.st,
                                                                           g.pd, g.dl) > 0);
+    const auto others = [&] { wgrad_rows_or_gather(dy, x, g, precision, out_type, o, gather); };
     if (rows) {
-        wgrad_rows_or_gather(dy, x, g, precision, out_type, o, gather);
+        others();
         return;
     }
-    auto ws = scratch((size_t)need);
-    check_k(nn_wgemm(x.type, out_type, o, x.data(), dy.data(), g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, cus, ws->ptr,
-                     need, stream()),
-            "convolve2_gradient_nn");
+    or_with_less_memory(
+        [&] {
+            auto ws = scratch((size_t)need);
+            check_k(nn_wgemm(x.type, out_type, o, x.data(), dy.data(), g.x.d, g.w.d, g.y.d, g.st, g.pd, g.dl, cus,
+                             ws->ptr, need, stream()),
+                    "convolve2_gradient_nn");
+        },
+        others);
 }
 
 // cpu::conv2FilterGradient<T>, src/backend/cpu/convolve.cpp:213-243

@@ -146,6 +146,7 @@ void *pool_alloc(size_t bytes) {
         (void)hipGetLastError();
         pool_gc();
         e = hipMalloc(&p, sz);
+        if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
     }
     check_hip(e, "hipMalloc");
     std::lock_guard<std::mutex> g(P.m);
