@@ -85,6 +85,46 @@ def test_values_out_of_range(af, rng, what, monkeypatch):
             np.testing.assert_allclose(a[fin], b[fin], rtol=2e-5, atol=2e-5)
 
 
+@pytest.mark.parametrize("split", ["2", "4"])
+@pytest.mark.parametrize("g", GEOMS, ids=_id)
+def test_split_reduction(af, rng, g, split, monkeypatch):
+    # partial tiles and their sum: phase padding, splits without slices in a
+    # phase without taps, columns past the last whole tile
+    x = rng.standard_normal(g[0]).astype(np.float32)
+    w = (rng.standard_normal(g[1]) * 0.1).astype(np.float32)
+    y64 = oracle.conv2_nn_direct_f64(x, w, *g[2:])
+    dy = rng.standard_normal(y64.shape).astype(np.float32)
+    dx64 = oracle.conv2_data_grad_direct_f64(dy, x, w, *g[2:])
+    monkeypatch.setenv("AFHIP_NN_X3", "1")
+    monkeypatch.setenv("AFHIP_NN_SPLIT", split)
+    for got, ref in zip(_both(af, af.Array(x), af.Array(w), af.Array(dy), g), (y64, dx64)):
+        assert oracle.rel_l2(got, ref) <= 5e-7
+        assert np.array_equal(got[ref == 0], ref[ref == 0])
+
+
+@pytest.mark.parametrize("split", ["2", "4"])
+def test_values_out_of_range_in_a_split(af, rng, split, monkeypatch):
+    # only the splits that read an infinity or a NaN run in FP32
+    g = ((30, 26, 70, 2), (3, 3, 70, 70), (1, 1), (1, 1), (1, 1))
+    x = rng.standard_normal(g[0]).astype(np.float32)
+    w = (rng.standard_normal(g[1]) * 0.1).astype(np.float32)
+    dy = rng.standard_normal((30, 26, 70, 2)).astype(np.float32)
+    for k, v in enumerate([np.inf, np.nan, -3e38, 1e12, -np.inf]):
+        x[3 * k, 25 - 3 * k, 5 * k, k % 2] = v
+        dy[29 - 3 * k, 3 * k, 8 * k, k % 2] = v
+    w[1, 1, 3, 7] = 1e11
+    X, W, DY = af.Array(x), af.Array(w), af.Array(dy)
+    monkeypatch.setenv("AFHIP_NN_X3", "1")
+    monkeypatch.setenv("AFHIP_NN_SPLIT", split)
+    got = _both(af, X, W, DY, g)
+    monkeypatch.setenv("AFHIP_NN_GATHER", "1")
+    for a, b in zip(got, _both(af, X, W, DY, g)):
+        np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
+        fin = np.isfinite(b)
+        np.testing.assert_array_equal(a[~fin & ~np.isnan(b)], b[~fin & ~np.isnan(b)])
+        np.testing.assert_allclose(a[fin], b[fin], rtol=2e-5, atol=2e-5)
+
+
 def test_tiny_values_among_others(af, rng, monkeypatch):
     # values far below the others (a saturated softmax's gradient) leave the
     # tile on the three parts: they add nothing to its sums but the side to
