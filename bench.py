@@ -5,7 +5,9 @@ gradient and for the filter gradient, on inputs already resident in HBM, for
 N=32 images of 64 channels at 56x56 with 128 filters of 3x3, stride 1, pad 1
 (the reference's convolve2_nn configuration). The timed arithmetic is BF16
 operands on the matrix cores with FP32 accumulation; the same step is also
-timed in FP32 (the plain path) for the BF16/FP32 ratio.
+timed in FP32 on the FP32 matrix instructions (the plain path) for the
+BF16/FP32 ratio, and in FP32 as the library runs it by default (three BF16 parts
+per operand).
 
 value = algorithmic FLOPs of (fwd + dgrad + wgrad) / step time, in TFLOP/s,
 where each pass counts 2*N*K*OH*OW*C*fh*fw FLOPs.
@@ -15,6 +17,7 @@ Prints ONE JSON line. --gpus N with N > 1 exits: this build runs one GPU.
 from __future__ import annotations
 
 import argparse
+import contextlib
 import ctypes
 import json
 import os
@@ -216,6 +219,44 @@ def time_af_api(af, ev, stream, X, W, DY, out_type, steps, warmup=2, precision=N
     ms = ev.ms(e0, e1) / steps
     del hold
     return ms
+
+
+@contextlib.contextmanager
+def fp32_plain():
+    """FP32 layers on the FP32 matrix instructions, in the patch and row-staged
+    kernels that NNStep runs through the kernel ABI."""
+    names = ("AFHIP_NN_X3", "AFHIP_NN_WG", "AFHIP_NN_SMALL")
+    before = {n: os.environ.get(n) for n in names}
+    os.environ.update({n: "0" for n in names})
+    try:
+        yield
+    finally:
+        for n, v in before.items():
+            if v is None:
+                del os.environ[n]
+            else:
+                os.environ[n] = v
+
+
+def time_passes(af, ev, stream, X, W, DY, steps, warmup):
+    """ms of each pass of the step through the af_* API."""
+    y = af.convolve2NN(X, W, ST, PD, DL)
+    passes = [lambda: af.convolve2NN(X, W, ST, PD, DL)] + [
+        lambda k=k: af.convolve2GradientNN(DY, X, W, y, ST, PD, DL, k)
+        for k in (af.AF_CONV_GRADIENT_DATA, af.AF_CONV_GRADIENT_FILTER)]
+    out = []
+    for p in passes:
+        for _ in range(warmup):
+            hold = p()
+        af.sync()
+        e0, e1 = ev.create(2)
+        ev.record(e0, stream)
+        for _ in range(steps):
+            hold = p()
+        ev.record(e1, stream)
+        out.append(ev.ms(e0, e1) / steps)
+        del hold
+    return out
 
 
 def time_graph(af, ev, stream, X, W, DY, steps, warmup):
@@ -758,8 +799,11 @@ def main():
     t0 = time.perf_counter()
     ms_bf16 = time_af_api(af, ev, stream, Xb, Wb, DYb, af.bf16, args.steps, args.warmup)
     wall_bf16 = time.perf_counter() - t0
-    ms_f32 = time_af_api(af, ev, stream, X32, W32, DY32, af.f32, max(3, args.steps // 2),
-                         max(1, args.warmup // 2))
+    n32, w32 = max(3, args.steps // 2), max(1, args.warmup // 2)
+    with fp32_plain():
+        ms_f32_plain = time_af_api(af, ev, stream, X32, W32, DY32, af.f32, n32, w32)
+    ms_f32 = time_af_api(af, ev, stream, X32, W32, DY32, af.f32, n32, w32)
+    per_f32_default = time_passes(af, ev, stream, X32, W32, DY32, n32, w32)
     # the same BF16 step as one captured hipGraph (afhip_nn_step_plan)
     ms_graph = time_graph(af, ev, stream, Xb, Wb, DYb, args.steps, args.warmup)
     # per-kernel durations: the same step through the kernel ABI with an event
@@ -768,9 +812,9 @@ def main():
     stepb = NNStep(af, Xb, Wb, DYb, af.bf16, af.bf16, af.PRECISION_DEFAULT)
     ms_kabi, kern_bf16, _ = time_step(af, ev, stream, stepb, args.steps, args.warmup)
     step32 = NNStep(af, X32, W32, DY32, af.f32, af.f32, af.PRECISION_DEFAULT)
-    _, kern_f32, _ = time_step(af, ev, stream, step32, max(3, args.steps // 2), max(1, args.warmup // 2))
+    _, kern_f32, _ = time_step(af, ev, stream, step32, n32, w32)
     tf_bf16 = 3 * flops_pass / (ms_bf16 * 1e-3) / 1e12
-    tf_f32 = 3 * flops_pass / (ms_f32 * 1e-3) / 1e12
+    tf_f32, tf_f32_plain = (3 * flops_pass / (t * 1e-3) / 1e12 for t in (ms_f32, ms_f32_plain))
     names = ["fwd", "dgrad", "wgrad"]
     per_bf16 = [sum(v for k, v in kern_bf16.items() if PASS_OF[k] == n) for n in names]
     per_f32 = [sum(v for k, v in kern_f32.items() if PASS_OF[k] == n) for n in names]
@@ -822,10 +866,13 @@ def main():
                    "global_batch": XD[3], "parallelism": "none (1 GPU)"},
         "ms_per_step_hipgraph": round(ms_graph, 4),
         "tflops_hipgraph": round(3 * flops_pass / (ms_graph * 1e-3) / 1e12, 3),
-        "fp32_plain_tflops": round(tf_f32, 3),
-        "bf16_over_fp32": round(tf_bf16 / tf_f32, 3),
+        "fp32_plain_tflops": round(tf_f32_plain, 3),
+        "bf16_over_fp32": round(tf_bf16 / tf_f32_plain, 3),
+        "fp32_default_tflops": round(tf_f32, 3),
+        "bf16_over_fp32_default": round(tf_bf16 / tf_f32, 3),
         "ms_per_pass_bf16": {n: round(float(v), 4) for n, v in zip(names, per_bf16)},
         "ms_per_pass_fp32": {n: round(float(v), 4) for n, v in zip(names, per_f32)},
+        "ms_per_pass_fp32_default": {n: round(float(v), 4) for n, v in zip(names, per_f32_default)},
         "us_per_kernel_bf16": {n: round(v * 1e3, 2) for n, v in kern_bf16.items()},
         "us_per_kernel_fp32": {n: round(v * 1e3, 2) for n, v in kern_f32.items()},
         "ms_per_step_bf16_kernel_abi_with_events": round(ms_kabi, 4),
