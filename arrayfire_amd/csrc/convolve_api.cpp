@@ -376,19 +376,20 @@ static bool whole_rows(const NNGeom &g, af_dtype t) {
 //    the GEMM (28x28x128x64 -> 128, 3x3: 171 and 121; 62x62x128x16 -> 128: 189
 //    and 145);
 //  * 16-bit: few channels (57x57x3x64 -> 64, 3x3: 37 and 44; to more than 32
-//    over odd rows the GEMM, 68x35x16x27 -> 128: 27 and 22), and whole rows
+//    over odd rows, or with more taps, the GEMM, 68x35x16x27 -> 128: 27 and 22;
+//    54x78x16x22 -> 16, 5x5, step: 127 and 101), and many whole rows
 //    under the weights-resident kernel or under pipelined stages that do not
 //    widen the channels (56x56x64x32 -> 128, 3x3: 29 and 39; 64x64x128x32 ->
 //    128, 1x1: 29 and 32; 32x32x96x64 -> 96, 5x5: 57 and 64). Else the GEMM
 //    (28x28x128x64 -> 128: 77 and 37; 48x48x64x64 -> 32, 5x5: 83 and 71;
 //    96x96x64x32 -> 64, 5x5, stride 2: 178 and 53; rows of 8 pixels 269 and
-//    110).
+//    110; 16x16x128x16 -> 96: 16.8 and 14.0).
 static bool patch_by_rule(int pass, const ArrayImpl &in, const NNGeom &g) {
     const dim_t R = pass == 0 ? g.x[2] : g.w[3], M = pass == 0 ? g.w[3] : g.x[2], taps = g.w[0] * g.w[1];
     const bool whole = whole_rows(g, in.type), unit = g.st[0] == 1 && g.st[1] == 1;
     if (in.type == f32) return whole && ((R > 8 && R <= 16) || (taps == 1 && R >= M));
-    if (R <= 8 || (R <= 16 && (whole || M <= 32))) return true;
-    if (!whole || g.x[0] < 16) return false;
+    if (taps <= 9 && (R <= 8 || (R <= 16 && (whole || M <= 32)))) return true;
+    if (!whole || g.x[0] < 16 || g.y[0] * g.y[1] * g.y[3] < 16384) return false;
     if (taps == 1) return unit && R >= M;
     return taps <= 9 ? unit || taps == 9 : unit && R >= 96;
 }
@@ -569,13 +570,13 @@ static void wgrad_rows_or_gather(const ArrayImpl &dy, const ArrayImpl &x, const 
 //    -> 64: 46 and 64; 32x32x256x32 -> 64, 1x1: 19 and 25). Else the GEMM
 //    (40x40x64x32 -> 64: 34 and 27; 56x56x16x32 -> 16: 36 and 29; 72x72x3x32 ->
 //    64: 53 and 46; 28x28x128x32 -> 128: 72 and 33; 72x70x48x3 -> 256: 35 and
-//    28; 80x80x256x4 -> 256, 1x1: 42 and 29).
+//    28; 32x66x32x22 -> 64: 30 and 23; 80x80x256x4 -> 256, 1x1: 42 and 29).
 static bool rows_by_rule(const ArrayImpl &x, const NNGeom &g) {
     if (!whole_rows(g, x.type)) return false;
     const dim_t lo = std::min(g.x[2], g.w[3]), hi = std::max(g.x[2], g.w[3]), px = g.y[0] * g.y[1] * g.y[3];
     const dim_t taps = g.w[0] * g.w[1], ow = g.y[0];
     if (x.type == f32) return taps == 1 && hi <= 64 && px >= 65536;
-    return px >= 32768 && hi >= 64 && lo >= 16 && ow >= 32 && ow * 5 >= (ow + 31) / 32 * 32 * 4 &&
+    return px >= 32768 && hi >= 64 && lo >= 16 && lo * hi * px >= 200000000 && ow >= 32 && ow * 5 >= (ow + 31) / 32 * 32 * 4 &&
            (taps > 1 || lo * hi * g.st[0] * g.st[1] <= 16384);
 }
 

@@ -18,8 +18,9 @@
 //    through the 8 linear-offset neighbours; the marked set is the closure of
 //    the seeds over weak pixels, computed here by repeated sweeps that mark a
 //    weak pixel next to a marked one, until a sweep changes nothing.
-// af_canny itself runs the tile kernels of canny_tiles.hip (and canny_otsu);
-// the kernels here are the steps one by one, for callers of the kernel ABI.
+// af_canny itself runs the tile kernels of canny_tiles.hip (and canny_otsu past
+// 4096 bins); the kernels here are the steps one by one, for callers of the
+// kernel ABI.
 // Arithmetic is uncontracted and in the reference's order, so every
 // comparison sees the reference's values.
 #include "kcommon.hpp"

@@ -945,12 +945,13 @@ __global__ __launch_bounds__(256) void nn_x3_copies(uint16_t *__restrict__ wp, c
 
 // As nn_clgemm, one 32-deep slice (three parts, 64 bytes each per row) per
 // stage, one LDS buffer and 64 x 64 tiles: four workgroups per CU cover each
-// other's loads, stores and barriers (a stage is 24 MFMAs per wave, the matrix
-// cores are busy about 40% of the time). x1w1 has accumulators of its own, so
+// other's loads, stores and barriers (a stage is 24 MFMAs per wave; the matrix
+// cores are busy 40% of the time, 34% in the data gradient). x1w1 has accumulators of its own, so
 // that the five small products, 2^-8 of it and below, are not rounded to its
 // last place each time; the two are added at the end. 56x56x64x32 -> 128, 3x3:
-// 112 us with the copies (19 us of them) against 139 us on the FP32 matrix
-// cores, its data gradient 134 against 153. Wider tiles (64 x 128: 117 us, 128 x
+// 114 us with the copies (14 us of them) against 139 us in nn_clgemm on the FP32
+// matrix cores, its data gradient 134 (25) against 153; where every tile runs in
+// FP32 (x and dy at 1e20 throughout), 283 and 305 us. Wider tiles (64 x 128: 117 us, 128 x
 // 128: 112 and 190 us) lose in occupancy what they save in LDS reads; two LDS
 // buffers with one barrier per stage cost a workgroup per CU (121 us).
 template <int PASS>

@@ -19,10 +19,10 @@
 // a block with huge values puts the parts together again and multiplies in FP32.
 //
 // us for the call, copies and sum included, against the kernels it replaces or
-// competes with (dims W H C N -> K): BF16 28x28x128x16 -> 128 3x3 stride 2: 20
-// (43, rows of 14 unaligned pixels), 55x47x64x8 -> 64 3x3: 19 (35),
-// 61x53x96x16 -> 32 5x5: 65 (455, element gather), 56x56x64x32 -> 128 3x3: 43
-// (45); FP32 the last one: 123 (207), error against FP64 2.2e-7 (5.1e-7).
+// competes with (dims W H C N -> K): BF16 28x28x128x16 -> 128 3x3 stride 2: 17
+// (37, rows of 14 unaligned pixels), 55x47x64x8 -> 64 3x3: 18 (38),
+// 61x53x96x16 -> 32 5x5: 51 (452, element gather), 56x56x64x32 -> 128 3x3: 49
+// (43); FP32 the last one: 123 (194), error against FP64 2.2e-7 (5.1e-7).
 // Bound by the loads of whole channel rows from L2 (each tap group reads its
 // pixels again) and, for FP32, by the six part products.
 #include <algorithm>
@@ -417,8 +417,12 @@ static bool wg_setup(int type, const long long *xd, const long long *wd, const l
     // 28x28x128x64 -> 128, 3x3, FP32: 42 splits (504 of 512) 113 us, 43 (516) 157.
     // The 16-bit kernels, of which four fit, take twice as many where each has
     // pixels enough (32x32x96x64 -> 96, 5x5: 97 us against 110; 28x28x128x64 ->
-    // 128, with 37 slices each of the larger share: 50 against 49).
-    const long long wide = !x3 && p->slices * ntile > 112LL * cus ? 4 : 2;
+    // 128, with 37 slices each of the larger share: 50 against 49) and half as many
+    // where there are few, for the fewer partials to write and sum (17x80x64x16 ->
+    // 128, 3x3: 23 us against 26; 21x70x3x34 -> 32, with 18 slices for each CU:
+    // 24 against 23).
+    const long long work = p->slices * ntile;
+    const long long wide = x3 ? 2 : work > 112LL * cus ? 4 : work < 18LL * cus ? 1 : 2;
     long long split = std::max<long long>(1, wide * cus / ntile);
     const long long each = (long long)p->RS * p->K * p->C * 4;
     split = std::min<long long>(split, (p->slices + 4 * SL - 1) / (4 * SL));  // at least four stages each

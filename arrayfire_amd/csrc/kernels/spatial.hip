@@ -672,8 +672,9 @@ __global__ __launch_bounds__(256) void conv2_whole(InT *__restrict__ out, const 
     }
 }
 
-// Square odd sides 3..9 (the halo of a larger one outgrows the tile); other
-// filters stay on conv_generic.
+// Square odd sides 3..9 are built; the halo of larger ones outgrows the tile, and
+// each even or oblong shape would be another seven instantiations: those stay on
+// conv_generic.
 template <typename InT>
 static int launch_whole(void *out, const void *in, const void *filt, const SpatialParams &p, hipStream_t s,
                         bool *served) {
@@ -724,9 +725,10 @@ struct Tile3Params {
 // flipped filter lives in SGPRs, for 5x5x5 two slices of it at a time (its 125
 // taps outnumber the SGPRs: kept whole, 115 were spilled to lanes of VGPRs,
 // 248 of which left two waves per SIMD). Bound by the FMAs, small volumes by one
-// round of workgroups. Before, with rows read as aligned float4s behind bounds
-// tests, and now: 192 x 190 x 128, 5x5x5 54.8 and 31.3 us (37 TFLOP/s); 256^3,
-// 5x5x5 179 and 91 us, 3x3x3 50 and 44 us; 128^3, 3x3x3 9.7 and 9.6 us.
+// round of workgroups that load, meet at a barrier, compute and store together.
+// Calls back to back, before, with rows read as aligned float4s behind bounds
+// tests, and now: 192 x 190 x 128, 5x5x5 55-57 and 29-33 us; 256^3, 5x5x5 180 and
+// 91-105 us, 3x3x3 50-53 and 44-46 us; 128^3, 3x3x3 9.5 and 9.0 us.
 constexpr int T3_BX = 32, T3_BY = 8, T3_BZ = 8;
 
 template <int FX, int FY, int FZ>
